@@ -349,6 +349,19 @@ int lmoe_grouped_down_f16w(const void *h, const uint32_t *offsets, const uint32_
                            int max_tiles, int bm, const void *wd16, int n_experts, int I, int H, void *y, int ydtype,
                            void *stream);
 
+/* lmoe_grouped_gate_up_f16w / lmoe_grouped_down_f16w straight from the blocks of one of the types Q4_1, Q8_0, Q5_K and
+ * Q6_K (gate and up of one type), decoded inside the GEMM with lmoe_dequant_gemm_f16's roundings: the same results bit
+ * for bit without the f16 copies. wg / wu [n_experts][I][row bytes], wd [n_experts][H][row bytes], aligned as that entry takes
+ * them (Q5_K 16 bytes, Q4_1 4, else 2); the contracted length a multiple of 128 (256 for Q5_K and Q6_K), I % 128, H % 256 for down; bm 128 or 64. R: down's rows
+ * (T topk). Replace the dense path's dequant + gather_mm on these types (gguf_experts.py:698-722; DEQ_SRC :529-539). */
+int lmoe_grouped_gate_up_any(const void *x, int xdtype, int T, int topk, const uint32_t *order,
+                             const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles,
+                             int bm, const uint8_t *wg, const uint8_t *wu, int type, int n_experts, int H, int I,
+                             void *h, void *stream);
+int lmoe_grouped_down_any(const void *h, int R, const uint32_t *offsets, const uint32_t *tiles,
+                          const uint32_t *n_tiles, int max_tiles, int bm, const uint8_t *wd, int type, int n_experts,
+                          int I, int H, void *y, int ydtype, void *stream);
+
 /* The trunk's 4-bit affine matmul of T bf16 rows: out [T][N] bf16 = x [T][K] bf16 . W^T with W in MLX's
  * affine 4-bit layout (w uint32 [N][K / 8], element j of a word at bits 4j; scales, biases bf16 [N][K / G];
  * weight = q s + b), each row with the bits of the reference's route_cuda.qmv_rows (route_cuda.py:460-541; MLX

@@ -25,10 +25,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CFLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off", "-Xclang", "-target-feature",
           "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function", "-Wno-unused-variable"]
 
-# Per-file extras. grouped.hip: MFMA accumulators in arch VGPRs. Left to its heuristics the compiler puts them in
+# Per-file extras. The grouped GEMMs: MFMA accumulators in arch VGPRs. Left to its heuristics the compiler puts them in
 # AGPRs with the untied MFMA form, and every K step then rotates them through ~130 accvgpr moves; in VGPRs they
 # stay put and the kernel fits two workgroups a CU (237 VGPRs, no AGPRs).
-FILE_FLAGS = {"grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+FILE_FLAGS = {n: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for n in ("grouped.hip", "grouped_any.hip")}
 
 
 def _run(cmd):

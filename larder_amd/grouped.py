@@ -128,6 +128,12 @@ def gemm_weights(w, t):
     return out
 
 
+def _decodes_in_gemm(t, K, bm):
+    """Whether the GEMMs decode type t's blocks themselves over a contraction of K (lmoe_grouped_*_any); else (a row that
+    does not split in steps of 128 weights) the blocks are dequantized to f16 first."""
+    return t not in _lib.Q4_TYPES and K % 128 == 0 and bm in (64, tile_rows())
+
+
 def _ws(n, ws, device):
     if n == 0:
         return None
@@ -153,9 +159,9 @@ def stream_copy(w, t):
 def gate_up(x, G, topk, wg, wu, types, h, xh=None, prepped=False, ws=None, ksplit=None, w16=None, sl=None):
     """h [R, I] f16 (grouped order, columns in the GEMMs' K order: from_kperm undoes it) = silu(x . wg) * (x . wu)
     over the grouping G of x's rows (row p reads x[order[p] // topk]); x [T, H] in natural order, any float dtype,
-    meets the weights as f16 in the K order (converted into ``xh``; prepped: x already is that form). Q4_0 / Q4_K
-    weights are decoded inside the GEMM; the other types are dequantized to f16 first (gemm_weights). ksplit
-    (None: pick_ksplit) and ws (the split-K workspace, allocated when not given) drive split-K. sl: (gate, up) in the
+    meets the weights as f16 in the K order (converted into ``xh``; prepped: x already is that form). Weights are
+    decoded inside the GEMM; gate and up of two types, or rows of a type beyond Q4_0 / Q4_K that do not split in steps
+    of 128 weights, are dequantized to f16 first (gemm_weights). ksplit (None: pick_ksplit) and ws (the split-K workspace, allocated when not given) drive split-K. sl: (gate, up) in the
     stream layout (stream_copy) to read instead of wg / wu, same results bit for bit."""
     tg, tu = qcode(types[0]), qcode(types[1])
     if not prepped:
@@ -169,6 +175,9 @@ def gate_up(x, G, topk, wg, wu, types, h, xh=None, prepped=False, ws=None, kspli
         entry, (wg_, wu_) = ("lmoe_grouped_gate_up_sl", sl) if sl is not None else ("lmoe_grouped_gate_up_bm", (wg, wu))
         call(entry, ptr(x), _lib.F16, T, topk, ptr(G.order), ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles),
              G.max_tiles, G.bm, ks, ptr(w), ptr(wg_), ptr(wu_), tg, tu, E, H, I, ptr(h), stream())
+    elif w16 is None and types[0] == types[1] and _decodes_in_gemm(types[0], H, G.bm):
+        call("lmoe_grouped_gate_up_any", ptr(x), _lib.F16, T, topk, ptr(G.order), ptr(G.offsets), ptr(G.tiles),
+             ptr(G.n_tiles), G.max_tiles, G.bm, ptr(wg), ptr(wu), tg, E, H, I, ptr(h), stream())
     else:
         if G.bm not in (64, tile_rows()):
             raise ValueError(f"the f16-weight GEMMs take 64- or {tile_rows()}-row tiles, not {G.bm}")
@@ -189,6 +198,9 @@ def down(h, G, wd, t, y, ws=None, ksplit=None, w16=None, sl=None):
         call("lmoe_grouped_down_sl" if sl is not None else "lmoe_grouped_down_bm", ptr(h), G.R, ptr(G.offsets),
              ptr(G.tiles), ptr(G.n_tiles), G.max_tiles, G.bm, ks, ptr(w), ptr(sl if sl is not None else wd), qcode(t),
              E, I, H, ptr(y), dcode(y.dtype), stream())
+    elif w16 is None and _decodes_in_gemm(t, I, G.bm):
+        call("lmoe_grouped_down_any", ptr(h), G.R, ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles), G.max_tiles, G.bm,
+             ptr(wd), qcode(t), E, I, H, ptr(y), dcode(y.dtype), stream())
     else:
         if G.bm not in (64, tile_rows()):
             raise ValueError(f"the f16-weight GEMMs take 64- or {tile_rows()}-row tiles, not {G.bm}")
