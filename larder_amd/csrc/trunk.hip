@@ -10,12 +10,16 @@
 // On gfx950 a 64-lane wavefront works two output rows, one a 32-lane half, so each half is exactly the reference's
 // warp and the butterfly stays inside the half (shuffles of width 32).
 //
-// bf16 arithmetic runs in float32 with gfx950's v_cvt_pk_bf16_f32 (round to nearest even) for each rounding:
-// products of two bf16 values are exact in float32; the sum of two bf16 values is exact unless their exponents
-// are more than 16 apart, where the small one cannot reach a bf16 rounding boundary. A fused multiply-add is one
-// float32 sum then one bf16 rounding; that double rounding equals the single rounding of the exact value except
-// when the float32 sum sits exactly on a bf16 midpoint with a nonzero error, where the error (recovered by TwoSum)
-// moves the sum off the midpoint first. (gfx950 has no bf16 fused multiply-add instruction.)
+// bf16 arithmetic runs in float32 with gfx950's v_cvt_pk_bf16_f32 (round to nearest even) for each rounding; with 0 as its
+// low operand the result is the rounded value as a float32 already, no unpacking. Products of two bf16 values are exact
+// in float32; the sum of two bf16 values is exact unless their exponents are more than 16 apart, where the small one
+// cannot reach a bf16 rounding boundary. gfx950 has no bf16 fused multiply-add: see fma_bf16_odd.
+//
+// VALU-bound (one product is 11-12 instructions, 5 of them the fused multiply-add's, against 0.56 bytes of weights).
+// Measured on one box, us, with the exact error of a nearest-rounded float32 sum recovered (TwoSum) and moved off the
+// bf16 midpoints (15 instructions) -> rounded to odd: 2048 -> 248,320 1 row 263 -> 157, 2048 -> 8192 1 row 12.2 -> 7.9,
+// 5 rows 37.6 -> 19.1, 2048 -> 512 5 rows 15.1 -> 8.7. Eight elements a mode change instead of sixteen: 566 against 495
+// at 248,320 x 5 rows, 173 against 166 at 1.
 #include "lmoe_common.h"
 
 namespace lmoe {
@@ -24,27 +28,68 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
-// both values rounded to bf16 by one v_cvt_pk_bf16_f32 (round to nearest even), back as float32
-__device__ __forceinline__ void bf16r2(float &a, float &b) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
-  a = __uint_as_float(u << 16);
-  b = __uint_as_float(u & 0xffff0000u);
+// v rounded to bf16 (nearest even), as float32
+__device__ __forceinline__ float bf16r(float v) {
+  return __uint_as_float(__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{0.0f, v}, bf16x2_t)));
 }
 
-
-// x w + a for bf16 values x, w, a as a float32 value whose round-to-nearest-even to bf16 is the single rounding
-// of the exact value: the float32 sum s and its exact error e (TwoSum; the product is exact); when s sits exactly
-// on a bf16 midpoint and e != 0, s moves one float32 ulp toward the exact value (it cannot cross another bf16
-// rounding boundary), so the conversion rounds the way the exact value does.
-__device__ __forceinline__ float fma_bf16_pre(float x, float w, float a) {
-  const float p = x * w;  // exact
-  const float s = p + a;
-  const float bb = s - p;
-  const float e = (p - (s - bb)) + (a - bb);  // s + e == p + a exactly
-  const uint32_t u = __float_as_uint(s);
-  const bool fix = (u & 0xffffu) == 0x8000u && e != 0.0f;
-  const uint32_t step = ((__float_as_uint(e) ^ u) >> 31) ? 0xffffffffu : 1u;  // away from zero when signs agree
-  return __uint_as_float(fix ? u + step : u);
+// a[i] <- x[i] w[i] + a[i] rounded to odd in float32 (the float32 neighbour of the exact value whose last bit is set,
+// unless the value is a float32 itself): a value whose rounding to bf16 is the one rounding of the exact value, since
+// only a value that is exactly halfway between two bf16 values ends in 0x8000. The exact value lies between the fused
+// multiply-add rounded down (MODE's round field = 2) and rounded up (1), which are equal or neighbours; the odd one is
+// picked bit by bit. One asm block, so that no other rounding instruction can come between the mode changes; the
+// smallest exact zero keeps the sign that rounding to nearest gives it (rounded up's +0, unless both are -0).
+__device__ __forceinline__ void fma_bf16_odd(float (&a)[16], const float *x, const float *w) {
+  float t[16];
+  asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
+      "v_fma_f32 %16, %32, %48, %0\n\t"
+      "v_fma_f32 %17, %33, %49, %1\n\t"
+      "v_fma_f32 %18, %34, %50, %2\n\t"
+      "v_fma_f32 %19, %35, %51, %3\n\t"
+      "v_fma_f32 %20, %36, %52, %4\n\t"
+      "v_fma_f32 %21, %37, %53, %5\n\t"
+      "v_fma_f32 %22, %38, %54, %6\n\t"
+      "v_fma_f32 %23, %39, %55, %7\n\t"
+      "v_fma_f32 %24, %40, %56, %8\n\t"
+      "v_fma_f32 %25, %41, %57, %9\n\t"
+      "v_fma_f32 %26, %42, %58, %10\n\t"
+      "v_fma_f32 %27, %43, %59, %11\n\t"
+      "v_fma_f32 %28, %44, %60, %12\n\t"
+      "v_fma_f32 %29, %45, %61, %13\n\t"
+      "v_fma_f32 %30, %46, %62, %14\n\t"
+      "v_fma_f32 %31, %47, %63, %15\n\t"
+      "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 1\n\t"
+      "v_fma_f32 %0, %32, %48, %0\n\t"
+      "v_fma_f32 %1, %33, %49, %1\n\t"
+      "v_fma_f32 %2, %34, %50, %2\n\t"
+      "v_fma_f32 %3, %35, %51, %3\n\t"
+      "v_fma_f32 %4, %36, %52, %4\n\t"
+      "v_fma_f32 %5, %37, %53, %5\n\t"
+      "v_fma_f32 %6, %38, %54, %6\n\t"
+      "v_fma_f32 %7, %39, %55, %7\n\t"
+      "v_fma_f32 %8, %40, %56, %8\n\t"
+      "v_fma_f32 %9, %41, %57, %9\n\t"
+      "v_fma_f32 %10, %42, %58, %10\n\t"
+      "v_fma_f32 %11, %43, %59, %11\n\t"
+      "v_fma_f32 %12, %44, %60, %12\n\t"
+      "v_fma_f32 %13, %45, %61, %13\n\t"
+      "v_fma_f32 %14, %46, %62, %14\n\t"
+      "v_fma_f32 %15, %47, %63, %15\n\t"
+      "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
+      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),
+        "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15]),
+        "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3]), "=&v"(t[4]), "=&v"(t[5]), "=&v"(t[6]), "=&v"(t[7]),
+        "=&v"(t[8]), "=&v"(t[9]), "=&v"(t[10]), "=&v"(t[11]), "=&v"(t[12]), "=&v"(t[13]), "=&v"(t[14]),
+        "=&v"(t[15])
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]),
+        "v"(x[9]), "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "v"(w[0]), "v"(w[1]),
+        "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]),
+        "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]), "v"(w[15]));
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int odd = __builtin_amdgcn_sbfe(__float_as_int(t[i]), 0, 1);  // all ones where rounded down is odd
+    asm("v_bfi_b32 %0, %1, %2, %0" : "+v"(a[i]) : "v"(odd), "v"(t[i]));
+  }
 }
 
 // Grid ceil(N / 8), 256 threads: wavefront w's lanes 0-31 work output row 8 bx + 2 w, lanes 32-63 the next one.
@@ -62,36 +107,36 @@ __global__ void __launch_bounds__(256) k_qmv_rows(const uint16_t *x, const uint3
   for (int r = 0; r < NR; ++r)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[r][e] = 0.0f;
-  for (int base = 0; base < K; base += 512) {
-    const int idx = base + 16 * l;
-    if (idx >= K) break;
+  // the lane's group: one division, then whole groups a 512-element step where G divides 512 (a division a step is 15 of
+  // a step's ~205 vector instructions)
+  const int gstep = 512 % G == 0 ? 512 / G : 0;
+  int grp = 16 * l / G;
+  for (int idx = 16 * l; idx < K; idx += 512, grp = gstep ? grp + gstep : idx / G) {
     const u32x2_t wv = *reinterpret_cast<const u32x2_t *>(wr + (idx >> 3));
-    const float s = bf16_to_f32(sr[idx / G]), b = bf16_to_f32(br[idx / G]);
+    const float s = bf16_to_f32(sr[grp]), b = bf16_to_f32(br[grp]);
     float wd[16];
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-      const uint32_t byte = ((p < 4 ? wv[0] : wv[1]) >> (8 * (p & 3))) & 0xffu;
-      float m0 = float(byte & 15u) * s, m1 = float(byte >> 4) * s;  // exact
-      bf16r2(m0, m1);
-      m0 += b;  // exact, or too far from a rounding boundary to matter
-      m1 += b;
-      bf16r2(m0, m1);
-      wd[2 * p] = m0;
-      wd[2 * p + 1] = m1;
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t lo = opaque(wv[h] & 0x0F0F0F0Fu), hi = opaque((wv[h] >> 4) & 0x0F0F0F0Fu);
+#pragma unroll
+      for (int p = 0; p < 8; ++p) {
+        const float m = bf16r(float(((p & 1 ? hi : lo) >> (8 * (p >> 1))) & 0xffu) * s);  // the product is exact
+        wd[8 * h + p] = bf16r(m + b);  // exact, or too far from a rounding boundary to matter
+      }
     }
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       const u32x4 *xp = reinterpret_cast<const u32x4 *>(x + size_t(r) * K + idx);
-      const u32x4 xa = xp[0], xc = xp[1];
-      const uint32_t xs[8] = {xa[0], xa[1], xa[2], xa[3], xc[0], xc[1], xc[2], xc[3]};
+      float xf[16];
 #pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        float s0 = fma_bf16_pre(__uint_as_float(xs[p] << 16), wd[2 * p], acc[r][2 * p]);
-        float s1 = fma_bf16_pre(__uint_as_float(xs[p] & 0xffff0000u), wd[2 * p + 1], acc[r][2 * p + 1]);
-        bf16r2(s0, s1);
-        acc[r][2 * p] = s0;
-        acc[r][2 * p + 1] = s1;
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 xs = xp[h];
+#pragma unroll
+        for (int p = 0; p < 8; ++p) xf[8 * h + p] = __uint_as_float(p & 1 ? xs[p >> 1] & 0xffff0000u : xs[p >> 1] << 16);
       }
+      fma_bf16_odd(acc[r], xf, wd);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[r][e] = bf16r(acc[r][e]);
     }
   }
 #pragma unroll
