@@ -362,6 +362,19 @@ int lmoe_grouped_down_any(const void *h, int R, const uint32_t *offsets, const u
                           const uint32_t *n_tiles, int max_tiles, int bm, const uint8_t *wd, int type, int n_experts,
                           int I, int H, void *y, int ydtype, void *stream);
 
+/* lmoe_grouped_down_bm (Q4_0, Q4_K; ksplit and ws as there) or lmoe_grouped_down_any (the other types, ksplit 1) with row p
+ * of the grouping written to row order[p] of out [R][H] in odtype (F32, F16, BF16): with one slot a row the experts'
+ * unweighted outputs in the caller's order, one rounding from the fp32 sums, without a pass to unsort them. Rows past
+ * offsets[n_experts] are not written (lmoe_rows_to_gemm_f16 clears them). Replaces the dense path's gather_mm down and its
+ * unsort (gguf_experts.py:720-722). */
+int lmoe_grouped_down_rows(const void *h, int R, const uint32_t *order, const uint32_t *offsets, const uint32_t *tiles,
+                           const uint32_t *n_tiles, int max_tiles, int bm, int ksplit, float *ws, const uint8_t *wd,
+                           int type_d, int n_experts, int I, int H, void *out, int odtype, void *stream);
+/* lmoe_to_gemm_f16 on rows x [R][H] into xh, and the rows of out [R][H] (odtype) whose ids [R] entry is past the experts
+ * set to zero, in one launch. H % 32 == 0. No counterpart in the reference (its slots are all valid). */
+int lmoe_rows_to_gemm_f16(const void *x, int xdtype, int R, int H, const uint32_t *ids, int n_experts, void *xh, void *out,
+                          int odtype, void *stream);
+
 /* The trunk's 4-bit affine matmul of T bf16 rows: out [T][N] bf16 = x [T][K] bf16 . W^T with W in MLX's
  * affine 4-bit layout (w uint32 [N][K / 8], element j of a word at bits 4j; scales, biases bf16 [N][K / G];
  * weight = q s + b), each row with the bits of the reference's route_cuda.qmv_rows (route_cuda.py:460-541; MLX

@@ -109,21 +109,36 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
   return __builtin_bit_cast(uint32_t, h2_t{_Float16(a), _Float16(b)});
 }
 
+// Two bf16 of a, b packed in one word (round to nearest even)
+__device__ __forceinline__ uint32_t pack_bf2(float a, float b) {
+  typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2_t{a, b}, bf2_t));
+}
+
 // acc[nb][mb][r] = D[tile feature frag_feature(nb) + 4 g + r][tile row 16 mb + fr]. Every store is 16 bytes:
 //   * gate/up: h (f16, K order) = silu(gate) * up. A lane's features 4g..4g+3 of fragments 0 and 1 (32 w + 4g.. and
 //     32 w + 16 + 4g.. of the n-tile) sit at K-order positions 8g..8g+3 and 8g+4..8g+7 of their 32-block: one store;
-//   * down, f16: fragments nb and nb + 1 meet through one permlane16 swap a word: lane group g then holds 8
+//   * down, 16-bit: fragments nb and nb + 1 meet through one permlane16 swap a word: lane group g then holds 8
 //     consecutive features, of fragment nb + (g & 1), from 8 (g >> 1) on, so a row's 32 features of the pair go out
 //     as one 64-byte run; f32: each fragment's 4 features as they are.
+// Down rows go to row p of out (grouped order), or with `order` to row order[p] (the caller's order, -0 stored as +0 as a
+// sum over one row's output would give it).
 // Called by every lane of the workgroup (the swaps read the lanes 16 away); rows past the tile's end store nothing.
-template <int MODE, int MB = 8>
-__device__ __forceinline__ void store_tile(f32x4 (&acc)[4][MB], const Tile &t, int wave, int fr, int g, void *out,
-                                           int ldo, int odt) {
+template <int MODE, bool ROWS, int MB>
+__device__ __forceinline__ void store_tile_as(f32x4 (&acc)[4][MB], const Tile &t, int wave, int fr, int g, void *out,
+                                              int ldo, int odt, const uint32_t *order) {
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     const int m = 16 * mb + fr;
     const bool ok = m < t.rows;
-    const size_t o = size_t(t.row0 + (ok ? m : 0)) * ldo;
+    size_t row = size_t(t.row0 + (ok ? m : 0));
+    if (ROWS) {
+      row = order[row];
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) acc[nb][mb] += 0.0f;
+    }
+    const size_t o = row * ldo;
     if (MODE == MODE_GATE_UP) {
       uint32_t v[4];
 #pragma unroll
@@ -142,20 +157,37 @@ __device__ __forceinline__ void store_tile(f32x4 (&acc)[4][MB], const Tile &t, i
                                      4 * g) = acc[nb][mb];
       }
     } else {
+      auto pack = [&](float a, float b) { return ROWS && odt == LMOE_BF16 ? pack_bf2(a, b) : pack_h2(a, b); };
 #pragma unroll
       for (int pr = 0; pr < 2; ++pr) {
         const int nb = 2 * pr;
-        const auto s0 = __builtin_amdgcn_permlane16_swap(pack_h2(acc[nb][mb][0], acc[nb][mb][1]),
-                                                         pack_h2(acc[nb + 1][mb][0], acc[nb + 1][mb][1]), false, false);
-        const auto s1 = __builtin_amdgcn_permlane16_swap(pack_h2(acc[nb][mb][2], acc[nb][mb][3]),
-                                                         pack_h2(acc[nb + 1][mb][2], acc[nb + 1][mb][3]), false, false);
+        const auto s0 = __builtin_amdgcn_permlane16_swap(pack(acc[nb][mb][0], acc[nb][mb][1]),
+                                                         pack(acc[nb + 1][mb][0], acc[nb + 1][mb][1]), false, false);
+        const auto s1 = __builtin_amdgcn_permlane16_swap(pack(acc[nb][mb][2], acc[nb][mb][3]),
+                                                         pack(acc[nb + 1][mb][2], acc[nb + 1][mb][3]), false, false);
         const uint32_t a0 = s0[0], b0 = s0[1], a1 = s1[0], b1 = s1[1];
         const int n = t.nt * GN + frag_feature<MODE>(wave, nb + (g & 1)) + 8 * (g >> 1);
-        if (ok) *reinterpret_cast<u32x4 *>(static_cast<_Float16 *>(out) + o + n) = u32x4{a0, a1, b0, b1};
+        if (ok) *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(out) + o + n) = u32x4{a0, a1, b0, b1};
       }
     }
   }
 }
+
+template <int MODE, int MB = 8>
+__device__ __forceinline__ void store_tile(f32x4 (&acc)[4][MB], const Tile &t, int wave, int fr, int g, void *out,
+                                           int ldo, int odt, const uint32_t *order) {
+  if (MODE == MODE_DOWN && order)  // uniform: one test a tile (tests a row block cost prompts 1-2%)
+    store_tile_as<MODE, true>(acc, t, wave, fr, g, out, ldo, odt, order);
+  else
+    store_tile_as<MODE, false>(acc, t, wave, fr, g, out, ldo, odt, order);
+}
+
+// The GEMMs that decode Q4_1 / Q8_0 / Q5_K / Q6_K (grouped_any.hip), shape checks included. mode gate/up: n_rows = I, a
+// gathered through order; down: n_rows = H, order the output rows (nullptr: grouped order).
+int grouped_any(const char *fn, int mode, const void *a, long long a_rows, int topk, const uint32_t *order,
+                const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles, int bm,
+                const uint8_t *w0, const uint8_t *w1, int type, int n_experts, int K, int n_rows, void *out, int odt,
+                hipStream_t st);
 
 // A wavefront-uniform pointer held in scalar registers (the copy instructions take their base there)
 template <typename P>

@@ -400,7 +400,7 @@ k_grouped_q4_0(const _Float16 *a_src, int topk, const uint32_t *order, const uin
     }
     return;
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // k_grouped_q4_0 on the GGUF layout with two-unit steps (K 128, the stage above): grid, arguments and results as
@@ -540,7 +540,7 @@ k_grouped_q4_0_w2(const _Float16 *a_src, int topk, const uint32_t *order, const 
     }
     return;
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // k_grouped_q4_0<MODE, GMT> on the GGUF layout for the tall tiles (128 or 64 rows, no split-K), with the weights
@@ -662,7 +662,7 @@ k_grouped_q4_0_p2(const _Float16 *a_src, int topk, const uint32_t *order, const 
       default: run(IC<4>{}); break;
     }
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // Finishes a split-K grouped GEMM: rows p < offsets[E] (the grouped rows of real experts), 4 features a thread:
@@ -670,7 +670,8 @@ k_grouped_q4_0_p2(const _Float16 *a_src, int topk, const uint32_t *order, const 
 // i .. i + 3 of I; down: y[p][n] (F16 / F32). Grid (ceil(N / 1024), R): N = I (gate/up) or H (down).
 template <int MODE>
 __global__ void __launch_bounds__(256) k_splitk_finish(const float *ws, int ksplit, int R, int ldw,
-                                                       const uint32_t *offsets, int E, void *out, int ldo, int odt) {
+                                                       const uint32_t *offsets, int E, void *out, int ldo, int odt,
+                                                       const uint32_t *order) {
   const int p = blockIdx.y;
   if (p >= int(offsets[E])) return;
   const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
@@ -682,7 +683,7 @@ __global__ void __launch_bounds__(256) k_splitk_finish(const float *ws, int kspl
     a += *reinterpret_cast<const f32x4 *>(row + n);
     if (MODE == MODE_GATE_UP) b += *reinterpret_cast<const f32x4 *>(row + N + n);
   }
-  const size_t o = size_t(p) * ldo;
+  const size_t o = size_t(order ? int(order[p]) : p) * ldo;
   if (MODE == MODE_GATE_UP) {
     const h2_t v01 = {_Float16(silu_mul_h(a[0], b[0])), _Float16(silu_mul_h(a[1], b[1]))};
     const h2_t v23 = {_Float16(silu_mul_h(a[2], b[2])), _Float16(silu_mul_h(a[3], b[3]))};
@@ -690,6 +691,8 @@ __global__ void __launch_bounds__(256) k_splitk_finish(const float *ws, int kspl
         u32x2{__builtin_bit_cast(uint32_t, v01), __builtin_bit_cast(uint32_t, v23)};
   } else if (odt == LMOE_F32) {
     *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + o + n) = a;
+  } else if (odt == LMOE_BF16) {
+    *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(out) + o + n) = u32x2{pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
   } else {
     const h2_t v01 = {_Float16(a[0]), _Float16(a[1])}, v23 = {_Float16(a[2]), _Float16(a[3])};
     *reinterpret_cast<u32x2 *>(static_cast<_Float16 *>(out) + o + n) =
@@ -813,7 +816,7 @@ k_grouped_f16w(const _Float16 *a_src, int topk, const uint32_t *order, const uin
       default: run(IC<4>{}); break;
     }
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // ---- Q4_K: register staging with repack --------------------------------------------------------------------------
@@ -984,7 +987,7 @@ k_grouped_q4_k(const _Float16 *a_src, int topk, const uint32_t *order, const uin
       default: run(IC<4>{}); break;
     }
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // ---- Q4_K: global -> LDS directly, four stages of 64-row tiles --------------------------------------------------
@@ -1180,7 +1183,7 @@ k_grouped_q4_k_dma(const _Float16 *a_src, int topk, const uint32_t *order, const
     case 3: run(IC<(MB >= 3 ? 3 : MB)>{}); break;
     default: run(IC<MB>{}); break;
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // k_grouped_q4_k_dma<MODE, 64> on the GGUF layout with the weights staged two steps at a time. A one-step stage
@@ -1351,7 +1354,7 @@ k_grouped_q4_k_w2(const _Float16 *a_src, int topk, const uint32_t *order, const 
     case 3: run(IC<3>{}); break;
     default: run(IC<MB>{}); break;
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // x [n] in dt -> f16 (round to nearest even), 8 elements a thread (vector loads when the whole range allows).
@@ -1374,6 +1377,17 @@ __global__ void __launch_bounds__(256) k_to_f16(const void *x, int dt, long long
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     if (i < cnt) out[i0 + i] = _Float16(load_elt(x, size_t(i0 + i), dt));
+}
+
+// k_to_f16's K-order form over rows of length H (a multiple of 32), each with an expert id, that also clears the rows of
+// out that no expert will write: a row with an id past the experts is zeros in out.
+__global__ void __launch_bounds__(256) k_rows_to_f16(const void *x, int dt, long long n, int H, const uint32_t *ids, int E,
+                                                     _Float16 *xh, void *out, int odt) {
+  to_f16_kperm(blockIdx.x, x, dt, n, xh);
+  const long long i0 = (static_cast<long long>(blockIdx.x) * 256 + threadIdx.x) * 8;
+  if (i0 >= n || ids[i0 / H] < uint32_t(E)) return;
+  const float z[8] = {};
+  store8(out, size_t(i0), odt, z);
 }
 
 // ---- the prefill router: logits = x . wr^T on the matrix cores ------------------------------------------------
@@ -1634,6 +1648,24 @@ extern "C" int lmoe_to_gemm_f16(const void *x, int xdtype, long long n, void *ou
   return to_f16("lmoe_to_gemm_f16", x, xdtype, n, out, stream, 1);
 }
 
+extern "C" int lmoe_rows_to_gemm_f16(const void *x, int xdtype, int R, int H, const uint32_t *ids, int n_experts, void *xh,
+                                     void *out, int odtype, void *stream) {
+  const char *fn = "lmoe_rows_to_gemm_f16";
+  LMOE_REQUIRE(dtype_ok(xdtype) && dtype_ok(odtype), LMOE_EINVAL, "%s: bad dtype", fn);
+  LMOE_REQUIRE(R >= 0 && H > 0 && H % 32 == 0 && n_experts > 0, LMOE_ESHAPE, "%s: %d rows of %d (a multiple of 32)", fn, R,
+               H);
+  if (R == 0) return 0;
+  LMOE_REQUIRE(x && ids && xh && out, LMOE_EINVAL, "%s: null pointer", fn);
+  LMOE_REQUIRE(aligned16(x) && aligned16(xh) && aligned16(out), LMOE_EALIGN, "%s: x, xh and out must be 16-byte aligned",
+               fn);
+  const long long n = (long long)R * H, blocks = (n + 2047) / 2048;
+  LMOE_REQUIRE(blocks < (1ll << 31), LMOE_ESHAPE, "%s: %lld elements", fn, n);
+  launch(k_rows_to_f16, dim3(unsigned(blocks)), dim3(256), 0, (hipStream_t)stream, x, xdtype, n, H, ids, n_experts,
+         static_cast<_Float16 *>(xh), out, odtype);
+  LMOE_LAUNCHED(fn);
+  return 0;
+}
+
 // ksplit > 1: the split-K form (32-row Q4_0 tiles): ksplit workgroups a tile, fp32 slices in ws, then
 // k_splitk_finish. Checks shared by both GEMMs.
 static int check_split(const char *fn, int bm, int type, int ksplit, const float *ws, int K, int R) {
@@ -1730,7 +1762,8 @@ static int grouped_gate_up(const char *fn, bool sl, const void *x, int xdtype, i
     if (ksplit > 1) {
       LMOE_LAUNCHED(fn);
       launch(k_splitk_finish<MODE_GATE_UP>, dim3(unsigned((I / 4 + 255) / 256), unsigned(R)), dim3(256), 0, st,
-             static_cast<const float *>(ws), ksplit, R, 2 * I, offsets, n_experts, h, I, int(LMOE_F16));
+             static_cast<const float *>(ws), ksplit, R, 2 * I, offsets, n_experts, h, I, int(LMOE_F16),
+             static_cast<const uint32_t *>(nullptr));
     }
   } else {
     launch(sl           ? k_grouped_q4_k_dma<MODE_GATE_UP, 64, 4, true>
@@ -1744,7 +1777,7 @@ static int grouped_gate_up(const char *fn, bool sl, const void *x, int xdtype, i
   return 0;
 }
 
-static int grouped_down(const char *fn, bool sl, const void *h, int R, const uint32_t *offsets,
+static int grouped_down(const char *fn, bool sl, const void *h, int R, const uint32_t *order, const uint32_t *offsets,
                         const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles, int bm, int ksplit, float *ws,
                         const uint8_t *wd, int type_d, int n_experts, int I, int H, void *y, int ydtype,
                         void *stream) {
@@ -1758,7 +1791,8 @@ static int grouped_down(const char *fn, bool sl, const void *h, int R, const uin
   LMOE_REQUIRE(I > 0 && I % block_weights(type_d) == 0 && I % 64 == 0, LMOE_ESHAPE,
                "%s: intermediate size %d is not a multiple of %d", fn, I, type_d == LMOE_Q4_K ? 256 : 64);
   LMOE_REQUIRE(H > 0 && H % GN == 0, LMOE_ESHAPE, "%s: hidden size %d is not a multiple of %d", fn, H, GN);
-  LMOE_REQUIRE(ydtype == LMOE_F16 || ydtype == LMOE_F32, LMOE_EINVAL, "%s: y must be float16 or float32", fn);
+  LMOE_REQUIRE(ydtype == LMOE_F16 || ydtype == LMOE_F32 || (order && ydtype == LMOE_BF16), LMOE_EINVAL,
+               "%s: y must be float16 or float32", fn);
   if (max_tiles == 0) return 0;
   LMOE_REQUIRE(h && offsets && tiles && n_tiles && wd && y, LMOE_EINVAL, "%s: null pointer", fn);
   LMOE_REQUIRE(aligned16(h) && aligned16(y) && aligned4(wd), LMOE_EALIGN,
@@ -1787,20 +1821,20 @@ static int grouped_down(const char *fn, bool sl, const void *h, int R, const uin
       kern = w2 == 2 ? k_grouped_q4_0_w2<MODE_DOWN, 32, 2> : k_grouped_q4_0_w2<MODE_DOWN, 32, 3>;
     if (q0_tall_pairs(sl, bm, I, ksplit))
       kern = bm == 64 ? k_grouped_q4_0_p2<MODE_DOWN, 64> : k_grouped_q4_0_p2<MODE_DOWN, GM>;
-    launch(kern, dim3(unsigned(grid)), dim3(kThreads), 0, st, a, 1, static_cast<const uint32_t *>(nullptr), offsets,
+    launch(kern, dim3(unsigned(grid)), dim3(kThreads), 0, st, a, 1, order, offsets,
            tiles, n_tiles, n_ntile, wd, static_cast<const uint8_t *>(nullptr), I, H, y, H, ydtype, ksplit, ws, R,
            H);
     if (ksplit > 1) {
       LMOE_LAUNCHED(fn);
       launch(k_splitk_finish<MODE_DOWN>, dim3(unsigned((H / 4 + 255) / 256), unsigned(R)), dim3(256), 0, st,
-             static_cast<const float *>(ws), ksplit, R, H, offsets, n_experts, y, H, ydtype);
+             static_cast<const float *>(ws), ksplit, R, H, offsets, n_experts, y, H, ydtype, order);
     }
   } else {
     launch(sl           ? k_grouped_q4_k_dma<MODE_DOWN, 64, 4, true>
            : bm == 32   ? k_grouped_q4_k<MODE_DOWN, 32, 3>
            : bm == 64   ? (qk_pairs() ? k_grouped_q4_k_w2<MODE_DOWN> : k_grouped_q4_k_dma<MODE_DOWN>)
                         : k_grouped_q4_k<MODE_DOWN>,
-           dim3(unsigned(grid)), dim3(kThreads), 0, st, a, 1, static_cast<const uint32_t *>(nullptr), offsets, tiles,
+           dim3(unsigned(grid)), dim3(kThreads), 0, st, a, 1, order, offsets, tiles,
            n_tiles, n_ntile, wd, static_cast<const uint8_t *>(nullptr), I, H, y, H, ydtype);
   }
   LMOE_LAUNCHED(fn);
@@ -1829,15 +1863,30 @@ extern "C" int lmoe_grouped_down_bm(const void *h, int R, const uint32_t *offset
                                     const uint32_t *n_tiles, int max_tiles, int bm, int ksplit, float *ws,
                                     const uint8_t *wd, int type_d, int n_experts, int I, int H, void *y, int ydtype,
                                     void *stream) {
-  return grouped_down("lmoe_grouped_down_bm", false, h, R, offsets, tiles, n_tiles, max_tiles, bm, ksplit, ws, wd,
+  return grouped_down("lmoe_grouped_down_bm", false, h, R, nullptr, offsets, tiles, n_tiles, max_tiles, bm, ksplit, ws, wd,
                       type_d, n_experts, I, H, y, ydtype, stream);
+}
+
+extern "C" int lmoe_grouped_down_rows(const void *h, int R, const uint32_t *order, const uint32_t *offsets,
+                                      const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles, int bm, int ksplit,
+                                      float *ws, const uint8_t *wd, int type_d, int n_experts, int I, int H, void *out,
+                                      int odtype, void *stream) {
+  const char *fn = "lmoe_grouped_down_rows";
+  LMOE_REQUIRE(order || max_tiles == 0, LMOE_EINVAL, "%s: null pointer", fn);
+  LMOE_REQUIRE(dtype_ok(odtype), LMOE_EINVAL, "%s: bad dtype", fn);
+  if (qtype_ok(type_d))
+    return grouped_down(fn, false, h, R, order, offsets, tiles, n_tiles, max_tiles, bm, ksplit, ws, wd, type_d, n_experts,
+                        I, H, out, odtype, stream);
+  LMOE_REQUIRE(ksplit == 1 && R >= 0, LMOE_ESHAPE, "%s: split-K takes 32-row Q4_0 tiles", fn);
+  return grouped_any(fn, MODE_DOWN, h, R, 1, order, offsets, tiles, n_tiles, max_tiles, bm, wd, nullptr, type_d, n_experts,
+                     I, H, out, odtype, (hipStream_t)stream);
 }
 
 extern "C" int lmoe_grouped_down_sl(const void *h, int R, const uint32_t *offsets, const uint32_t *tiles,
                                     const uint32_t *n_tiles, int max_tiles, int bm, int ksplit, float *ws,
                                     const uint8_t *wd, int type_d, int n_experts, int I, int H, void *y, int ydtype,
                                     void *stream) {
-  return grouped_down("lmoe_grouped_down_sl", true, h, R, offsets, tiles, n_tiles, max_tiles, bm, ksplit, ws, wd,
+  return grouped_down("lmoe_grouped_down_sl", true, h, R, nullptr, offsets, tiles, n_tiles, max_tiles, bm, ksplit, ws, wd,
                       type_d, n_experts, I, H, y, ydtype, stream);
 }
 

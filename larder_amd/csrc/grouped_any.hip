@@ -352,11 +352,11 @@ k_grouped_any(const _Float16 *a_src, int topk, const uint32_t *order, const uint
     case 3: run(IC<3>{}); break;
     default: run(IC<4>{}); break;
   }
-  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt);
+  store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
 // Shape checks and the launch both entry points share. mode gate/up: n_rows = I; down: n_rows = H.
-static int grouped_any(const char *fn, int mode, const void *a, long long a_rows, int topk, const uint32_t *order,
+int grouped_any(const char *fn, int mode, const void *a, long long a_rows, int topk, const uint32_t *order,
                        const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles, int bm,
                        const uint8_t *w0, const uint8_t *w1, int type, int n_experts, int K, int n_rows, void *out,
                        int odt, hipStream_t st) {

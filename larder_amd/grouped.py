@@ -221,11 +221,23 @@ def expert_rows(x, w, host, types, out_dtype):
     ids = torch.as_tensor(host).reshape(-1).to(device=dev, dtype=torch.int32)
     G = Grouping(R, E, dev, bm=pick_tile_rows(R, E, types)).run(ids)
     h = torch.empty((R, I), dtype=torch.float16, device=dev)
+    out = torch.empty((R, H), dtype=out_dtype, device=dev)
+    t = types[2]
+    if t in _lib.Q4_TYPES or _decodes_in_gemm(t, I, G.bm):  # down writes the caller's rows itself
+        x = x.contiguous()
+        xh = torch.empty((R, H), dtype=torch.float16, device=dev)
+        call("lmoe_rows_to_gemm_f16", ptr(x), dcode(x.dtype), R, H, ptr(ids.contiguous()), E, ptr(xh), ptr(out),
+             dcode(out_dtype), stream())
+        gate_up(xh, G, 1, wg, wu, types, h, prepped=True)
+        ks = pick_ksplit(R, E, G.bm, I) if t == "Q4_0" else 1
+        ws = _ws(ks * R * H if ks > 1 else 0, None, dev)
+        call("lmoe_grouped_down_rows", ptr(h), R, ptr(G.order), ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles), G.max_tiles,
+             G.bm, ks, ptr(ws), ptr(wd), qcode(t), E, I, H, ptr(out), dcode(out_dtype), stream())
+        return out
     # the down GEMM's f32 result goes to out_dtype with one rounding: an f16 y only when out is f16 itself
     y = torch.empty((R, H), dtype=torch.float16 if out_dtype == torch.float16 else torch.float32, device=dev)
     gate_up(x.contiguous(), G, 1, wg, wu, types, h)
-    down(h, G, wd, types[2], y)
-    out = torch.empty((R, H), dtype=out_dtype, device=dev)
+    down(h, G, wd, t, y)
     call("lmoe_combine_sorted", ptr(y), dcode(y.dtype), ptr(G.inv), None, R, 1, H, None, None, 0, None, 0, ptr(out),
          dcode(out_dtype), stream())
     bad = (ids < 0) | (ids >= E)
