@@ -67,6 +67,11 @@ int lmoe_timeline_clock_khz(int *khz);
 int lmoe_router_topk(const void *logits, int ldtype, int T, int E, int k, int norm, uint32_t *ids, float *scores,
                      void *stream);
 
+/* lmoe_router_topk with each token's picks in ascending rank, best last: the layout of route_cuda.probs
+ * (route_cuda.py:230-233, 280-288). */
+int lmoe_router_probs(const void *logits, int ldtype, int T, int E, int k, int norm, uint32_t *ids, float *scores,
+                      void *stream);
+
 /* lmoe_router_topk and lmoe_to_gemm_f16 in ONE launch (no counterpart in the reference; the prefill chain's two steps
  * before the grouping when the logits are given, stream_fast.py:4352-4370 / gguf_experts.py:698-722): ids / scores
  * [T][k] from logits [T][E] as lmoe_router_topk gives them, and x [n] (n % 32 == 0, 16-byte aligned) to xh [n] in f16
@@ -388,6 +393,12 @@ int lmoe_qmv_rows(const void *x, int T, const uint32_t *w, const void *scales, c
  * leaves it to MLX ops, whose bf16 bits are not reproduced here). */
 int lmoe_swiglu_bf16(const void *g, const void *u, long long n, void *out, void *stream);
 
+/* lmoe_qmv_rows for two weights of one shape (gate, up) and lmoe_swiglu_bf16 of the two in one launch, the same bits:
+ * out [T][N] bf16 = bf16(silu(g) u). */
+int lmoe_qmv_swiglu_rows(const void *x, int T, const uint32_t *wg, const void *scales_g, const void *biases_g,
+                         const uint32_t *wu, const void *scales_u, const void *biases_u, int N, int K, int group_size,
+                         void *out, void *stream);
+
 /* x [n] (F32 / BF16 / F16) -> out [n] float16, round to nearest even.
  * No counterpart in the reference (its dense path casts with MLX, gguf_experts.py:716). */
 int lmoe_to_f16(const void *x, int xdtype, long long n, void *out, void *stream);
@@ -449,6 +460,11 @@ int lmoe_router_gemm_refine(const void *xh, int T, int H, const void *wk, int E,
 int lmoe_combine_sorted(const void *y, int ydtype, const uint32_t *inv, const float *scores, int T, int k, int H,
                         const float *shared, const float *gate, int gate_stride, const void *residual,
                         int rdtype, void *out, int odtype, void *stream);
+
+/* lmoe_combine_sorted on rows in the caller's order (y [T][k][H], row t k + j of token t) with the shared rows [T][H] and
+ * gate logits [T] in dtypes of their own (read as fp32): route_cuda.tail (route_cuda.py:290-298) in one launch. */
+int lmoe_combine_rows(const void *y, int ydtype, const float *scores, int T, int k, int H, const void *shared, int sdtype,
+                      const void *gate, int gdtype, void *out, int odtype, void *stream);
 
 /* Experts at `slots` of buf [S][rows][row bytes] as dense weights q [n][rows][cols] in odtype (F16, BF16, F32).
  * Replaces gguf_experts.dequant (gguf_experts.py:579-586; kernel gguf_dequant :529-539). */

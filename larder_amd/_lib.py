@@ -99,6 +99,9 @@ SIGNATURES = {
     "lmoe_grouped_down_any": (_I, [_P, _I, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P, _I, _P]),
     "lmoe_grouped_down_rows": (_I, [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _P, _I, _I, _I, _I, _P, _I, _P]),
     "lmoe_rows_to_gemm_f16": (_I, [_P, _I, _I, _I, _P, _I, _P, _P, _I, _P]),
+    "lmoe_router_probs": (_I, [_P, _I, _I, _I, _I, _I, _P, _P, _P]),
+    "lmoe_combine_rows": (_I, [_P, _I, _P, _I, _I, _I, _P, _I, _P, _I, _P, _I, _P]),
+    "lmoe_qmv_swiglu_rows": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P, _P]),
     "lmoe_quantize_q4_0": (_I, [_P, _I, _LL, _I, _P, _P]),
     "lmoe_quantize_q4_k": (_I, [_P, _I, _LL, _I, _P, _P]),
 }

@@ -1,47 +1,66 @@
 // Smaller kernels around the path: the weighted combine of grouped rows, the dequant of whole experts, and a
 // Q4_0 quantizer used to build synthetic packs on the device.
+#include <type_traits>
+
 #include "lmoe_common.h"
 
 namespace lmoe {
 
 // out[t][n] = sum_j scores[t][j] y[inv[t k + j]][n] (+ sigmoid(gate) shared) (+ residual), in that order of
-// additions; VEC: 8 consecutive n a thread (H % 8 == 0, aligned rows), grid (ceil(H / 2048), T); else one n a
-// thread, grid (ceil(H / 256), T).
+// additions; inv null: row t k + j. VEC: 8 consecutive n a thread (H % 8 == 0, aligned rows), grid (ceil(H / 2048), T);
+// else one n a thread, grid (ceil(H / 256), T). Bound by y's bytes at a prompt's size (8,192 tokens x 8 rows of 2048:
+// 58 us, 5.2 TB/s) and by its round trips at a few tokens, so the rows' loads go out 8 (then 4, 2, 1) at a time.
 template <bool VEC>
 __global__ void __launch_bounds__(256)
     k_combine_sorted(const void *y, int ydt, const uint32_t *inv, const float *scores, int k, int H,
-                     const float *shared, const float *gate, int gate_stride, const void *residual, int rdt,
-                     void *out, int odt) {
+                     const void *shared, int sdt, const void *gate, int gdt, int gate_stride, const void *residual,
+                     int rdt, void *out, int odt) {
   const int t = blockIdx.y;
   constexpr int NV = VEC ? 8 : 1;
   const int n = (blockIdx.x * 256 + threadIdx.x) * NV;
   if (n >= H) return;
+  auto load = [&](const void *p, size_t i, int dt, float *v) {
+    if (VEC)
+      load8(p, i, dt, v);
+    else
+      v[0] = load_elt(p, i, dt);
+  };
   float acc[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) acc[i] = 0.0f;
-  for (int j = 0; j < k; ++j) {
-    const size_t row = inv[size_t(t) * k + j];
-    const float s = scores ? scores[size_t(t) * k + j] : 1.0f;
-    float v[NV];
-    if (VEC)
-      load8(y, row * H + n, ydt, v);
-    else
-      v[0] = load_elt(y, row * H + n, ydt);
+  auto rows = [&](int j0, auto nc) {  // rows j0 .. j0 + N - 1
+    constexpr int N = decltype(nc)::value;
+    float v[N][NV], s[N];
+    size_t row[N];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) acc[i] = fmaf(s, v[i], acc[i]);
-  }
+    for (int j = 0; j < N; ++j) {
+      const size_t at = size_t(t) * k + j0 + j;
+      row[j] = inv ? inv[at] : at;
+      s[j] = scores ? scores[at] : 1.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) load(y, row[j] * H + n, ydt, v[j]);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) acc[i] = fmaf(s[j], v[j][i], acc[i]);
+  };
+  int j = 0;
+  for (; j + 8 <= k; j += 8) rows(j, std::integral_constant<int, 8>{});
+  if (k - j >= 4) rows(j, std::integral_constant<int, 4>{}), j += 4;
+  if (k - j >= 2) rows(j, std::integral_constant<int, 2>{}), j += 2;
+  if (k - j >= 1) rows(j, std::integral_constant<int, 1>{});
   const size_t o = size_t(t) * H + n;
   if (shared) {
-    const float gs = sigmoidf_(gate[size_t(t) * gate_stride]);
+    const float gs = sigmoidf_(load_elt(gate, size_t(t) * gate_stride, gdt));
+    float v[NV];
+    load(shared, o, sdt, v);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) acc[i] += gs * shared[o + i];
+    for (int i = 0; i < NV; ++i) acc[i] += gs * v[i];
   }
   if (residual) {
     float v[NV];
-    if (VEC)
-      load8(residual, o, rdt, v);
-    else
-      v[0] = load_elt(residual, o, rdt);
+    load(residual, o, rdt, v);
 #pragma unroll
     for (int i = 0; i < NV; ++i) acc[i] += v[i];
   }
@@ -187,26 +206,39 @@ __global__ void __launch_bounds__(256) k_quantize_q4_k(const void *w, int wdt, l
 
 using namespace lmoe;
 
+static int combine(const char *fn, const void *y, int ydtype, const uint32_t *inv, const float *scores, int T, int k,
+                   int H, const void *shared, int sdtype, const void *gate, int gdtype, int gate_stride,
+                   const void *residual, int rdtype, void *out, int odtype, void *stream) {
+  LMOE_REQUIRE(dtype_ok(ydtype) && dtype_ok(odtype) && (!residual || dtype_ok(rdtype)) &&
+                   (!shared || (dtype_ok(sdtype) && dtype_ok(gdtype))),
+               LMOE_EINVAL, "%s: bad dtype", fn);
+  LMOE_REQUIRE(T >= 0 && k > 0 && H > 0, LMOE_ESHAPE, "%s: bad shape", fn);
+  LMOE_REQUIRE(!shared == !gate, LMOE_EINVAL, "%s: shared and gate go together", fn);
+  if (T == 0) return 0;
+  LMOE_REQUIRE(y && out, LMOE_EINVAL, "%s: null pointer", fn);
+  const bool vec = H % 8 == 0 && aligned16(y) && aligned16(out) && (!residual || aligned16(residual)) &&
+                   (!shared || aligned16(shared)) &&
+                   (ydtype != LMOE_F32 || (reinterpret_cast<uintptr_t>(y) & 31u) == 0);
+  launch(vec ? k_combine_sorted<true> : k_combine_sorted<false>, dim3(vec ? (H + 2047) / 2048 : (H + 255) / 256, T),
+         dim3(256), 0, (hipStream_t)stream, y, ydtype, inv, scores, k, H, shared, sdtype, gate, gdtype, gate_stride,
+         residual, rdtype, out, odtype);
+  LMOE_LAUNCHED(fn);
+  return 0;
+}
+
 extern "C" int lmoe_combine_sorted(const void *y, int ydtype, const uint32_t *inv, const float *scores, int T, int k,
                                    int H, const float *shared, const float *gate, int gate_stride,
                                    const void *residual, int rdtype, void *out, int odtype, void *stream) {
   const char *fn = "lmoe_combine_sorted";
-  LMOE_REQUIRE(dtype_ok(ydtype) && dtype_ok(odtype) && (!residual || dtype_ok(rdtype)), LMOE_EINVAL,
-               "%s: bad dtype", fn);
-  LMOE_REQUIRE(T >= 0 && k > 0 && H > 0, LMOE_ESHAPE, "%s: bad shape", fn);
-  LMOE_REQUIRE(!shared == !gate, LMOE_EINVAL, "%s: shared and gate go together", fn);
-  if (T == 0) return 0;
-  LMOE_REQUIRE(y && inv && out, LMOE_EINVAL, "%s: null pointer", fn);
-  const bool vec = H % 8 == 0 && aligned16(y) && aligned16(out) && (!residual || aligned16(residual)) &&
-                   (ydtype != LMOE_F32 || (reinterpret_cast<uintptr_t>(y) & 31u) == 0);
-  if (vec)
-    launch(k_combine_sorted<true>, dim3((H + 2047) / 2048, T), dim3(256), 0, (hipStream_t)stream, y, ydtype, inv,
-           scores, k, H, shared, gate, gate_stride, residual, rdtype, out, odtype);
-  else
-    launch(k_combine_sorted<false>, dim3((H + 255) / 256, T), dim3(256), 0, (hipStream_t)stream, y, ydtype, inv,
-           scores, k, H, shared, gate, gate_stride, residual, rdtype, out, odtype);
-  LMOE_LAUNCHED(fn);
-  return 0;
+  LMOE_REQUIRE(inv || T <= 0, LMOE_EINVAL, "%s: null pointer", fn);
+  return combine(fn, y, ydtype, inv, scores, T, k, H, shared, LMOE_F32, gate, LMOE_F32, gate_stride, residual, rdtype,
+                 out, odtype, stream);
+}
+
+extern "C" int lmoe_combine_rows(const void *y, int ydtype, const float *scores, int T, int k, int H, const void *shared,
+                                 int sdtype, const void *gate, int gdtype, void *out, int odtype, void *stream) {
+  return combine("lmoe_combine_rows", y, ydtype, nullptr, scores, T, k, H, shared, sdtype, gate, gdtype, 1, nullptr, 0, out,
+                 odtype, stream);
 }
 
 extern "C" int lmoe_dequant(const uint8_t *buf, int type, int n_experts, int rows, int cols, const uint32_t *slots,

@@ -21,7 +21,8 @@ constexpr int kMaxNpl = 16;  // logits a lane: E <= 64 * 16
 // Four tokens a workgroup, one wavefront each (k_router_topk's body).
 template <int NPL>
 __device__ __forceinline__ void topk_rows(int block, const void *logits, int ldt, int ld_stride, int T, int E,
-                                          int k, int norm, uint32_t *ids, float *scores, const float *gate, int m) {
+                                          int k, int norm, uint32_t *ids, float *scores, const float *gate, int m,
+                                          int best_last = 0) {
   __shared__ __attribute__((aligned(16))) uint32_t scr[4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = block * 4 + wave;
@@ -38,8 +39,9 @@ __device__ __forceinline__ void topk_rows(int block, const void *logits, int ldt
   topk_wave<NPL>(v, E, k, norm, scr[wave], &id, &sc);
   const int ks = k + m;
   if (lane < k) {
-    ids[size_t(t) * ks + lane] = id;
-    scores[size_t(t) * ks + lane] = sc;
+    const int at = best_last ? k - 1 - lane : lane;
+    ids[size_t(t) * ks + at] = id;
+    scores[size_t(t) * ks + at] = sc;
   } else if (lane < ks) {
     ids[size_t(t) * ks + lane] = uint32_t(E + lane - k);
     scores[size_t(t) * ks + lane] = sigmoidf_(gate[t]);
@@ -52,8 +54,8 @@ __device__ __forceinline__ void topk_rows(int block, const void *logits, int ldt
 template <int NPL>
 __global__ void __launch_bounds__(256) k_router_topk(const void *logits, int ldt, int ld_stride, int T, int E,
                                                      int k, int norm, uint32_t *ids, float *scores,
-                                                     const float *gate = nullptr, int m = 0) {
-  topk_rows<NPL>(blockIdx.x, logits, ldt, ld_stride, T, E, k, norm, ids, scores, gate, m);
+                                                     const float *gate, int m, int best_last) {
+  topk_rows<NPL>(blockIdx.x, logits, ldt, ld_stride, T, E, k, norm, ids, scores, gate, m, best_last);
 }
 
 // The prefill's top-k and x's conversion to f16 in the GEMM K order (the two steps before the grouping that do not
@@ -633,7 +635,8 @@ __global__ void __launch_bounds__(1024) k_route_bias(RouteArgs a) {
 using namespace lmoe;
 
 static int topk_launch(const void *logits, int ldtype, int stride, int T, int E, int k, int norm, uint32_t *ids,
-                       float *scores, hipStream_t st, const char *fn, const float *gate = nullptr, int m = 0) {
+                       float *scores, hipStream_t st, const char *fn, const float *gate = nullptr, int m = 0,
+                       int best_last = 0) {
   LMOE_REQUIRE(dtype_ok(ldtype), LMOE_EINVAL, "%s: logits dtype %d is not F32, F16 or BF16", fn, ldtype);
   LMOE_REQUIRE(T >= 0 && E > 0 && E <= 64 * kMaxNpl, LMOE_ESHAPE, "%s: %d experts is outside 1..%d", fn, E,
                64 * kMaxNpl);
@@ -642,15 +645,15 @@ static int topk_launch(const void *logits, int ldtype, int stride, int T, int E,
   LMOE_REQUIRE(logits && ids && scores, LMOE_EINVAL, "%s: null pointer", fn);
   const dim3 grid((T + 3) / 4), block(256);
   if (E <= 64)
-    launch(k_router_topk<1>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m);
+    launch(k_router_topk<1>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m, best_last);
   else if (E <= 128)
-    launch(k_router_topk<2>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m);
+    launch(k_router_topk<2>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m, best_last);
   else if (E <= 256)
-    launch(k_router_topk<4>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m);
+    launch(k_router_topk<4>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m, best_last);
   else if (E <= 512)
-    launch(k_router_topk<8>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m);
+    launch(k_router_topk<8>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m, best_last);
   else
-    launch(k_router_topk<16>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m);
+    launch(k_router_topk<16>, grid, block, 0, st, logits, ldtype, stride, T, E, k, norm, ids, scores, gate, m, best_last);
   LMOE_LAUNCHED(fn);
   return 0;
 }
@@ -658,6 +661,11 @@ static int topk_launch(const void *logits, int ldtype, int stride, int T, int E,
 extern "C" int lmoe_router_topk(const void *logits, int ldtype, int T, int E, int k, int norm, uint32_t *ids,
                                 float *scores, void *stream) {
   return topk_launch(logits, ldtype, E, T, E, k, norm, ids, scores, (hipStream_t)stream, "lmoe_router_topk");
+}
+
+extern "C" int lmoe_router_probs(const void *logits, int ldtype, int T, int E, int k, int norm, uint32_t *ids,
+                                 float *scores, void *stream) {
+  return topk_launch(logits, ldtype, E, T, E, k, norm, ids, scores, (hipStream_t)stream, "lmoe_router_probs", nullptr, 0, 1);
 }
 
 extern "C" int lmoe_topk_and_gemm_f16(const void *logits, int ldtype, int T, int E, int k, int norm, uint32_t *ids,

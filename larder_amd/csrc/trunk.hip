@@ -20,6 +20,8 @@
 // bf16 midpoints (15 instructions) -> rounded to odd: 2048 -> 248,320 1 row 263 -> 157, 2048 -> 8192 1 row 12.2 -> 7.9,
 // 5 rows 37.6 -> 19.1, 2048 -> 512 5 rows 15.1 -> 8.7. Eight elements a mode change instead of sixteen: 566 against 495
 // at 248,320 x 5 rows, 173 against 166 at 1.
+#include <type_traits>
+
 #include "lmoe_common.h"
 
 namespace lmoe {
@@ -92,16 +94,11 @@ __device__ __forceinline__ void fma_bf16_odd(float (&a)[16], const float *x, con
   }
 }
 
-// Grid ceil(N / 8), 256 threads: wavefront w's lanes 0-31 work output row 8 bx + 2 w, lanes 32-63 the next one.
-// x [NR][K] bf16, out [NR][N] bf16. K % 16 == 0, G % 16 == 0, K % G == 0.
+// sum[r] = row r of x [NR][K] bf16 times one weight row (wr, sr, br), by the 32 lanes l of a half-wavefront, in every lane.
+// K % 16 == 0, G % 16 == 0, K % G == 0.
 template <int NR>
-__global__ void __launch_bounds__(256) k_qmv_rows(const uint16_t *x, const uint32_t *w, const uint16_t *scales,
-                                                  const uint16_t *biases, int N, int K, int G, uint16_t *out) {
-  const int lane = threadIdx.x & 63, l = lane & 31;
-  const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 2 + (lane >> 5);
-  const int rr = row < N ? row : N - 1;  // a half past N works the last row again and stores nothing
-  const uint32_t *wr = w + size_t(rr) * (K / 8);
-  const uint16_t *sr = scales + size_t(rr) * (K / G), *br = biases + size_t(rr) * (K / G);
+__device__ __forceinline__ void qmv_dot(const uint16_t *x, const uint32_t *wr, const uint16_t *sr, const uint16_t *br, int K,
+                                        int G, int l, float (&sum)[NR]) {
   float acc[NR][16];
 #pragma unroll
   for (int r = 0; r < NR; ++r)
@@ -146,7 +143,44 @@ __global__ void __launch_bounds__(256) k_qmv_rows(const uint16_t *x, const uint3
     for (int e = 0; e < 16; ++e) s += acc[r][e];
 #pragma unroll
     for (int m = 16; m > 0; m >>= 1) s += __shfl_xor(s, m, 32);
-    if (l == 0 && row < N) out[size_t(r) * N + row] = f32_to_bf16(s);
+    sum[r] = s;
+  }
+}
+
+// Grid ceil(N / 8), 256 threads: wavefront w's lanes 0-31 work output row 8 bx + 2 w, lanes 32-63 the next one.
+// x [NR][K] bf16, out [NR][N] bf16.
+template <int NR>
+__global__ void __launch_bounds__(256) k_qmv_rows(const uint16_t *x, const uint32_t *w, const uint16_t *scales,
+                                                  const uint16_t *biases, int N, int K, int G, uint16_t *out) {
+  const int lane = threadIdx.x & 63, l = lane & 31;
+  const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 2 + (lane >> 5);
+  const int rr = row < N ? row : N - 1;  // a half past N works the last row again and stores nothing
+  float s[NR];
+  qmv_dot<NR>(x, w + size_t(rr) * (K / 8), scales + size_t(rr) * (K / G), biases + size_t(rr) * (K / G), K, G, l, s);
+  if (l == 0 && row < N) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) out[size_t(r) * N + row] = f32_to_bf16(s[r]);
+  }
+}
+
+// out [NR][N] bf16 = bf16(silu(g) u), g and u the bf16 products of two weights of one shape: grid ceil(N / 4), wavefront w's
+// lanes 0-31 work row 4 bx + w of the first weight, lanes 32-63 that row of the second (k_qmv_rows twice and
+// k_swiglu_bf16 in one launch, the same bits: at one token each of the three is a launch's latency).
+template <int NR>
+__global__ void __launch_bounds__(256) k_qmv_swiglu(const uint16_t *x, const uint32_t *wg, const uint16_t *sg,
+                                                    const uint16_t *bg, const uint32_t *wu, const uint16_t *su,
+                                                    const uint16_t *bu, int N, int K, int G, uint16_t *out) {
+  const int lane = threadIdx.x & 63, l = lane & 31;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= N) return;  // uniform across the wavefront
+  const bool up = lane >= 32;
+  const size_t gi = size_t(row) * (K / G);
+  float s[NR];
+  qmv_dot<NR>(x, (up ? wu : wg) + size_t(row) * (K / 8), (up ? su : sg) + gi, (up ? bu : bg) + gi, K, G, l, s);
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const float u = __shfl(s[r], 32);
+    if (lane == 0) out[size_t(r) * N + row] = f32_to_bf16(silu_mul(bf16r(s[r]), bf16r(u)));
   }
 }
 
@@ -174,40 +208,55 @@ extern "C" int lmoe_swiglu_bf16(const void *g, const void *u, long long n, void 
   return 0;
 }
 
-extern "C" int lmoe_qmv_rows(const void *x, int T, const uint32_t *w, const void *scales, const void *biases, int N,
-                             int K, int group_size, void *out, void *stream) {
-  const char *fn = "lmoe_qmv_rows";
+// The checks and the passes over x both products share: at most 8 rows a launch (their accumulators stay in registers);
+// rows 8.. in a second pass over the weights, which changes no bit (each row's arithmetic is its own). go(NR, first row).
+template <typename F>
+static int qmv_passes(const char *fn, const void *x, int T, const void *w, int N, int K, int group_size, F &&go) {
   LMOE_REQUIRE(T >= 0, LMOE_ESHAPE, "%s: %d rows", fn, T);
   LMOE_REQUIRE(N > 0 && K > 0 && K % 16 == 0 && group_size > 0 && group_size % 16 == 0 && K % group_size == 0,
                LMOE_ESHAPE, "%s: K %d and group size %d must be multiples of 16, K of the group size", fn, K,
                group_size);
   if (T == 0) return 0;
-  LMOE_REQUIRE(x && w && scales && biases && out, LMOE_EINVAL, "%s: null pointer", fn);
+  LMOE_REQUIRE(x && w, LMOE_EINVAL, "%s: null pointer", fn);
   LMOE_REQUIRE(aligned16(x) && (reinterpret_cast<uintptr_t>(w) & 7u) == 0, LMOE_EALIGN,
                "%s: x must be 16-byte aligned, w 8-byte aligned", fn);
-  const dim3 grid(unsigned((N + 7) / 8));
-  hipStream_t st = (hipStream_t)stream;
-  // at most 8 rows a launch (their accumulators stay in registers); rows 8.. in a second pass over the weights,
-  // which changes no bit (each row's arithmetic is its own)
   for (int r0 = 0; r0 < T; r0 += 8) {
-    const int nr = T - r0 < 8 ? T - r0 : 8;
-    const uint16_t *xr = static_cast<const uint16_t *>(x) + size_t(r0) * K;
-    uint16_t *orow = static_cast<uint16_t *>(out) + size_t(r0) * N;
-    auto go = [&](auto kern) {
-      launch(kern, grid, dim3(256), 0, st, xr, w, static_cast<const uint16_t *>(scales),
-             static_cast<const uint16_t *>(biases), N, K, group_size, orow);
-    };
-    switch (nr) {
-      case 1: go(k_qmv_rows<1>); break;
-      case 2: go(k_qmv_rows<2>); break;
-      case 3: go(k_qmv_rows<3>); break;
-      case 4: go(k_qmv_rows<4>); break;
-      case 5: go(k_qmv_rows<5>); break;
-      case 6: go(k_qmv_rows<6>); break;
-      case 7: go(k_qmv_rows<7>); break;
-      default: go(k_qmv_rows<8>); break;
+    switch (T - r0 < 8 ? T - r0 : 8) {
+      case 1: go(std::integral_constant<int, 1>{}, r0); break;
+      case 2: go(std::integral_constant<int, 2>{}, r0); break;
+      case 3: go(std::integral_constant<int, 3>{}, r0); break;
+      case 4: go(std::integral_constant<int, 4>{}, r0); break;
+      case 5: go(std::integral_constant<int, 5>{}, r0); break;
+      case 6: go(std::integral_constant<int, 6>{}, r0); break;
+      case 7: go(std::integral_constant<int, 7>{}, r0); break;
+      default: go(std::integral_constant<int, 8>{}, r0); break;
     }
     LMOE_LAUNCHED(fn);
   }
   return 0;
+}
+
+extern "C" int lmoe_qmv_rows(const void *x, int T, const uint32_t *w, const void *scales, const void *biases, int N,
+                             int K, int group_size, void *out, void *stream) {
+  const char *fn = "lmoe_qmv_rows";
+  LMOE_REQUIRE(T <= 0 || (scales && biases && out), LMOE_EINVAL, "%s: null pointer", fn);
+  return qmv_passes(fn, x, T, w, N, K, group_size, [&](auto nr, int r0) {
+    launch(k_qmv_rows<decltype(nr)::value>, dim3(unsigned((N + 7) / 8)), dim3(256), 0, (hipStream_t)stream,
+           static_cast<const uint16_t *>(x) + size_t(r0) * K, w, static_cast<const uint16_t *>(scales),
+           static_cast<const uint16_t *>(biases), N, K, group_size, static_cast<uint16_t *>(out) + size_t(r0) * N);
+  });
+}
+
+extern "C" int lmoe_qmv_swiglu_rows(const void *x, int T, const uint32_t *wg, const void *scales_g, const void *biases_g,
+                                    const uint32_t *wu, const void *scales_u, const void *biases_u, int N, int K,
+                                    int group_size, void *out, void *stream) {
+  const char *fn = "lmoe_qmv_swiglu_rows";
+  LMOE_REQUIRE(T <= 0 || (scales_g && biases_g && wu && scales_u && biases_u && out), LMOE_EINVAL, "%s: null pointer", fn);
+  LMOE_REQUIRE(T <= 0 || (reinterpret_cast<uintptr_t>(wu) & 7u) == 0, LMOE_EALIGN, "%s: w must be 8-byte aligned", fn);
+  return qmv_passes(fn, x, T, wg, N, K, group_size, [&](auto nr, int r0) {
+    launch(k_qmv_swiglu<decltype(nr)::value>, dim3(unsigned((N + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+           static_cast<const uint16_t *>(x) + size_t(r0) * K, wg, static_cast<const uint16_t *>(scales_g),
+           static_cast<const uint16_t *>(biases_g), wu, static_cast<const uint16_t *>(scales_u),
+           static_cast<const uint16_t *>(biases_u), N, K, group_size, static_cast<uint16_t *>(out) + size_t(r0) * N);
+  });
 }

@@ -14,17 +14,17 @@ last k of an ascending ranking (best expert last, route_cuda.py:230-233).
 """
 import torch
 
-from ._lib import call, dcode, ptr, stream
+from ._lib import DTYPE_CODE, call, dcode, ptr, stream
 
 
-def topk(logits, k, norm):
+def topk(logits, k, norm, entry="lmoe_router_topk"):
     """logits (..., E) -> (ids int32 (..., k) best first, scores float32 (..., k))."""
     lg = logits.contiguous()
     E = lg.shape[-1]
     T = lg.numel() // E
     ids = torch.empty(lg.shape[:-1] + (k,), dtype=torch.int32, device=lg.device)
     scores = torch.empty(lg.shape[:-1] + (k,), dtype=torch.float32, device=lg.device)
-    call("lmoe_router_topk", ptr(lg), dcode(lg.dtype), T, E, k, int(bool(norm)), ptr(ids), ptr(scores), stream())
+    call(entry, ptr(lg), dcode(lg.dtype), T, E, k, int(bool(norm)), ptr(ids), ptr(scores), stream())
     return ids, scores
 
 
@@ -32,8 +32,12 @@ def probs(logits, k, norm):
     """softmax(logits) then the top k, as route_cuda.probs returns them (route_cuda.py:280-288): inds int32
     (..., k) in ascending rank (best last) and their float32 softmax probabilities, renormalised to sum 1 when
     ``norm``."""
-    ids, scores = topk(logits, k, norm)
-    return ids.flip(-1).contiguous(), scores.flip(-1).contiguous()
+    return topk(logits, k, norm, "lmoe_router_probs")
+
+
+def _floats(t):
+    """t contiguous, in a dtype the kernels read as float32 (any other converted to it)."""
+    return (t if t.dtype in DTYPE_CODE else t.to(torch.float32)).contiguous()
 
 
 def tail(y, scores, shared, gate):
@@ -41,15 +45,13 @@ def tail(y, scores, shared, gate):
     scores (..., T, k), shared (..., T, D) float32 or None, gate (..., T, 1) or None; out in y's dtype."""
     t, k, d = y.shape[-3:]
     yy = y.reshape(t * k, d).contiguous()
-    inv = torch.arange(t * k, dtype=torch.int32, device=y.device)
     sc = scores.reshape(t, k).to(torch.float32).contiguous()
     out = torch.empty(y.shape[:-2] + (d,), dtype=y.dtype, device=y.device)
     sh = gt = None
     if shared is not None:
-        sh = shared.reshape(t, d).to(torch.float32).contiguous()
-        gt = gate.reshape(t).to(torch.float32).contiguous()
-    call("lmoe_combine_sorted", ptr(yy), dcode(yy.dtype), ptr(inv), ptr(sc), t, k, d, ptr(sh), ptr(gt), 1, None, 0,
-         ptr(out), dcode(out.dtype), stream())
+        sh, gt = _floats(shared.reshape(t, d)), _floats(gate.reshape(t))
+    call("lmoe_combine_rows", ptr(yy), dcode(yy.dtype), ptr(sc), t, k, d, ptr(sh), dcode(sh.dtype) if sh is not None else 0,
+         ptr(gt), dcode(gt.dtype) if gt is not None else 0, ptr(out), dcode(out.dtype), stream())
     return out
 
 

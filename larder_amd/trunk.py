@@ -45,6 +45,15 @@ def shared_expert_rows(x, gate, up, down):
     """mlx_lm's shared-expert MLP, down(silu(gate(x)) * up(x)), for x [..., T, H] bf16 with each projection a
     (w, scales, biases, group_size) 4-bit affine weight run through qmv_rows; the SwiGLU rounds once to bf16
     (lmoe_swiglu_bf16). The sigmoid-gated add to the routed output is route.tail's."""
+    (wg, sg, bg, gs), (wu, su, bu, us) = gate, up
+    if gs == us and wg.shape == wu.shape and qmv_fits(x, wg, sg, gs, 4, "affine", bg) and qmv_fits(
+            x, wu, su, us, 4, "affine", bu):  # gate, up and the SwiGLU in one launch
+        K, N = x.shape[-1], wg.shape[0]
+        x2 = x.reshape(-1, K).contiguous()
+        h = torch.empty((x2.shape[0], N), dtype=torch.bfloat16, device=x.device)
+        call("lmoe_qmv_swiglu_rows", ptr(x2), x2.shape[0], *(ptr(t.contiguous()) for t in (wg, sg, bg, wu, su, bu)), N, K, gs,
+             ptr(h), stream())
+        return qmv_rows(h.reshape(x.shape[:-1] + (N,)), *down)
     g = qmv_rows(x, *gate)
     u = qmv_rows(x, *up)
     h = torch.empty_like(g)

@@ -1,0 +1,56 @@
+"""GPU tests of the drop-in block's one-launch steps against the launches they stand for: the shared expert's gate, up and
+SwiGLU (lmoe_qmv_swiglu_rows), probs' best-last order (lmoe_router_probs) and tail (lmoe_combine_rows)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import qmv
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(rng, N, K, G):
+    wq, s, b = qmv.quantize_affine4((rng.standard_normal((N, K)) * 0.05).astype(np.float32), G)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda().bfloat16()  # noqa: E731
+    return torch.from_numpy(wq.view(np.int32)).cuda(), d(s), d(b), G
+
+
+@pytest.mark.parametrize("T,N,K,G", [(1, 512, 2048, 64), (3, 33, 528, 16), (8, 5, 64, 32), (9, 64, 1056, 48)])
+def test_qmv_swiglu_same_bits(T, N, K, G):
+    from larder_amd import trunk
+    from larder_amd._lib import call, ptr, stream
+    rng = np.random.default_rng(T + N)
+    gate, up = _weight(rng, N, K, G), _weight(rng, N, K, G)
+    x = torch.from_numpy(rng.standard_normal((T, K)).astype(np.float32)).cuda().bfloat16()
+    g, u = trunk.qmv_rows(x, *gate), trunk.qmv_rows(x, *up)
+    want = torch.empty_like(g)
+    call("lmoe_swiglu_bf16", ptr(g), ptr(u), g.numel(), ptr(want), stream())
+    got = torch.empty_like(g)
+    call("lmoe_qmv_swiglu_rows", ptr(x), T, *(ptr(t) for t in gate[:3] + up[:3]), N, K, G, ptr(got), stream())
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 256, 8), (5, 512, 10), (4, 60, 4), (67, 9, 9), (3, 1024, 32)])
+def test_probs_is_topk_reversed(T, E, k):
+    from larder_amd import route
+    lg = torch.randn((T, E), generator=torch.Generator(device="cuda").manual_seed(E), device="cuda").bfloat16()
+    ids, sc = route.topk(lg, k, True)
+    inds, scores = route.probs(lg, k, True)
+    assert torch.equal(inds, ids.flip(-1)) and torch.equal(scores, sc.flip(-1))
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 7, 8, 11, 15, 16])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
+def test_tail_every_row_count_and_dtype(k, dt):
+    """Any count of rows a token (groups of 8, 4, 2 and 1), aligned and odd widths, shared rows and gates in any dtype."""
+    from larder_amd import route
+    g = torch.Generator(device="cuda").manual_seed(k)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    for D in (64, 2056, 33):
+        y, sc, sh, gate = r(3, k, D).to(dt), r(3, k), r(3, D).to(dt), r(3, 1).to(dt)
+        want = (y.double() * sc.double()[..., None]).sum(-2)
+        tol = {torch.float32: 1e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[dt]  # one rounding of the output
+        for shared in (None, sh):
+            w = want if shared is None else want + torch.sigmoid(gate.double()) * sh.double()
+            got = route.tail(y, sc, shared, None if shared is None else gate).double()
+            assert float((got - w).norm() / w.norm()) < tol
