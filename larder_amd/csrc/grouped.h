@@ -35,37 +35,41 @@ enum { MODE_GATE_UP = 0, MODE_DOWN = 1 };
 __device__ __forceinline__ int achunk(int r, int c) { return r * 8 + (c ^ (r & 7)); }
 
 
-// two f16 (1024 + q) from a byte-wise masked word: {q0, q1} or {q2, q3}
+// two f16 (1024 + byte) from a word's bytes: {b0, b1} or {b2, b3}
 __device__ __forceinline__ uint32_t magic_pair(uint32_t nib, uint32_t sel) {
   return __builtin_amdgcn_perm(0x64646464u, nib, sel);
 }
 constexpr uint32_t kSel01 = 0x04010400u, kSel23 = 0x04030402u;
 
+// Bytes 0, 1 (HI false) or 2, 3 of a word of nibbles (0 .. 15 a byte) as f16, exactly: read as fp8 (E4M3), 0 .. 7 are the
+// subnormals n 2^-9 and 8 .. 15 the first binade (8 + m) 2^-9, so the conversion scaled by 2^9 gives the nibble. One
+// instruction (4 cycles a SIMD, like each of the byte permute and the packed subtraction that it stands for).
+template <bool HI>
+__device__ __forceinline__ h2_t nibbles_f16(uint32_t v) {
+  return __builtin_bit_cast(h2_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 512.0f, HI));
+}
+
 // An MFMA lane's 8 f16 weights from its nibble word x (low nibbles: K positions 0-3 of the lane group, high
-// nibbles: 4-7). Q4_0: w = ((1024 + q) - 1032) d, d = the selected half of sw. Q4_K: sw = {f16(d sc), f16(dmin m)},
-// w = fma((1024 + q) - 1024, d sc, -dmin m) (q exact, one rounding).
+// nibbles: 4-7), one rounding a weight. Q4_0: w = fma(q, d, -8 d), d = the selected half of sw (8 d is exact up to
+// |d| = 8188; a block past it has weights that no f16 holds). Q4_K: sw = {f16(d sc), f16(dmin m)}, w = fma(q, d sc,
+// -dmin m).
 template <int TB>
 __device__ __forceinline__ half8 decode8(uint32_t x, uint32_t sw, int half) {
   const uint32_t lo = x & 0x0F0F0F0Fu, hi = (x >> 4) & 0x0F0F0F0Fu;
-  const h2_t p[4] = {__builtin_bit_cast(h2_t, magic_pair(lo, kSel01)), __builtin_bit_cast(h2_t, magic_pair(lo, kSel23)),
-                     __builtin_bit_cast(h2_t, magic_pair(hi, kSel01)), __builtin_bit_cast(h2_t, magic_pair(hi, kSel23))};
-  h2_t bias, scale, sub;
+  const h2_t q[4] = {nibbles_f16<false>(lo), nibbles_f16<true>(lo), nibbles_f16<false>(hi), nibbles_f16<true>(hi)};
+  h2_t scale, add;
   if (TB == LMOE_Q4_0) {
-    const _Float16 d = __builtin_bit_cast(h2_t, sw)[half];
-    bias = h2_t{_Float16(1032.0f), _Float16(1032.0f)};
+    const _Float16 d = __builtin_bit_cast(h2_t, sw)[half], m8d = d * _Float16(-8.0f);
     scale = h2_t{d, d};
-    sub = h2_t{_Float16(0.0f), _Float16(0.0f)};
+    add = h2_t{m8d, m8d};
   } else {
     const h2_t v = __builtin_bit_cast(h2_t, sw);
-    bias = h2_t{_Float16(1024.0f), _Float16(1024.0f)};
     scale = h2_t{v[0], v[0]};
-    sub = h2_t{v[1], v[1]};
+    add = h2_t{-v[1], -v[1]};
   }
   uint32_t o[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    o[i] = TB == LMOE_Q4_0 ? __builtin_bit_cast(uint32_t, (p[i] - bias) * scale)
-                           : __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(p[i] - bias, scale, -sub));
+  for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q[i], scale, add));
   return __builtin_bit_cast(half8, u32x4{o[0], o[1], o[2], o[3]});
 }
 

@@ -38,21 +38,9 @@ __device__ __forceinline__ void byte_pairs(uint32_t a, uint32_t b, h2_t *p) {
   p[3] = __builtin_bit_cast(h2_t, magic_pair(b, kSel23));
 }
 
-// f16(float32(q s + c)) a weight: the product is exact, the sum rounds to float32, then to f16 (lmoe_dequant's steps;
-// v_fma_mixlo_f16 would round once, which differs in about one weight of 10 million)
-__device__ __forceinline__ half8 fma_pairs(const h2_t *q, const float *s, const float *c) {
-  half8 w;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float v = fmaf(float(q[i >> 1][i & 1]), s[i >> 2], c[i >> 2]);
-    asm("" : "+v"(v));  // keeps the sum and its conversion apart
-    w[i] = _Float16(v);
-  }
-  return w;
-}
-
-// f16(q s + c) a weight where q s + c is exact in float32: one instruction a weight. A half-register write needs a wait
-// state before its register is read: the low halves go first, and s_nop stands after the last.
+// f16(q s + c) for the 4 bytes q of a (s[0], c[0]) and of b (s[1], c[1]), given as f16 1024 + q pairs with c less 1024 s,
+// where the result is exact in float32: one instruction a weight. A half-register write needs a wait state before its
+// register is read: the low halves go first, and s_nop stands after the last.
 __device__ __forceinline__ half8 fma_pairs_exact(const h2_t *q, const float *s, const float *c) {
   uint32_t o[4];
   asm("v_fma_mixlo_f16 %0, %4, %8, %10 op_sel_hi:[1,0,0]\n\t"
@@ -69,6 +57,20 @@ __device__ __forceinline__ half8 fma_pairs_exact(const h2_t *q, const float *s, 
         "v"(__builtin_bit_cast(uint32_t, q[2])), "v"(__builtin_bit_cast(uint32_t, q[3])), "v"(s[0]), "v"(s[1]),
         "v"(c[0]), "v"(c[1]));
   return half8_of(o);
+}
+
+// f16(float32(q s + c)) for the 4 bytes q of a (s[0], c[0]) and of b (s[1], c[1]): the product is exact, the sum rounds to
+// float32, then to f16 (lmoe_dequant's steps; v_fma_mixlo_f16 would round once, which differs in about one weight of 10
+// million).
+__device__ __forceinline__ half8 fma_bytes(uint32_t a, uint32_t b, const float *s, const float *c) {
+  half8 w;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float v = fmaf(float(((i < 4 ? a : b) >> (8 * (i & 3))) & 0xffu), s[i >> 2], c[i >> 2]);
+    asm("" : "+v"(v));  // keeps the sum and its conversion apart
+    w[i] = _Float16(v);
+  }
+  return w;
 }
 
 constexpr int AK = 128;  // K a step
@@ -132,13 +134,8 @@ template <int H> struct Frag<LMOE_Q4_1, H> {
   __device__ __forceinline__ Frag(const uint8_t *rec, int g_) : r(rec), g(g_) {}
   __device__ __forceinline__ half8 weights(int j) const {  // f16(q d + m)
     const uint32_t dm = lds32(r + 20 * j), q = lds32(r + 20 * j + 4 + 4 * g);
-    h2_t p[4];
-    byte_pairs(q & 0x0F0F0F0Fu, (q >> 4) & 0x0F0F0F0Fu, p);
-    const h2_t bias = {_Float16(1024.0f), _Float16(1024.0f)};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] -= bias;
     const float s[2] = {half_lo(dm), half_lo(dm)}, c[2] = {half_hi(dm), half_hi(dm)};
-    return fma_pairs(p, s, c);
+    return fma_bytes(opaque(q & 0x0F0F0F0Fu), opaque((q >> 4) & 0x0F0F0F0Fu), s, c);
   }
 };
 
@@ -159,16 +156,11 @@ template <int H> struct Frag<LMOE_Q5_K, H> {  // header 16, qh 32, the half's qs
     for (int i = 0; i < 2; ++i)
       v[i] = ((lds32(r + 32 * (j >> 1) + 16 * i) >> (4 * (j & 1))) & 0x0F0F0F0Fu) |
              (((hb[i] >> sb) & 0x01010101u) << 4);
-    h2_t p[4];
-    byte_pairs(v[0], v[1], p);
-    const h2_t bias = {_Float16(1024.0f), _Float16(1024.0f)};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] -= bias;
     float sc, mn;
     k4_scale_min(hdr[1], hdr[2], hdr[3], sb, &sc, &mn);
     const float d1 = half_lo(hdr[0]) * sc, m1 = -(half_hi(hdr[0]) * mn);
     const float s[2] = {d1, d1}, c[2] = {m1, m1};
-    return fma_pairs(p, s, c);
+    return fma_bytes(opaque(v[0]), opaque(v[1]), s, c);
   }
 };
 
@@ -189,12 +181,12 @@ template <int H> struct Frag<LMOE_Q6_K, H> {  // the half's ql 64, qh 32, scales
     for (int i = 0; i < 2; ++i)
       v[i] = ((lds32(r + 32 * (j & 1) + 16 * i) >> (4 * (j >> 1))) & 0x0F0F0F0Fu) |
              (((hb[i] >> (2 * j)) & 0x03030303u) << 4);
-    h2_t p[4];
-    byte_pairs(v[0], v[1], p);
-    // (1024 + q) s - 1056 s: 1056 s (24 bits) and the result (24 bits) are exact in float32, so only f16 rounds
     const uint32_t sw = sc[j >> 1] >> (16 * (j & 1));
     const float s[2] = {d * float(int(int8_t(uint8_t(sw)))), d * float(int(int8_t(uint8_t(sw >> 8))))};
+    // (1024 + q) s - 1056 s: 1056 s (24 bits) and the result (24 bits) are exact in float32, so only f16 rounds
     const float c[2] = {-1056.0f * s[0], -1056.0f * s[1]};
+    h2_t p[4];
+    byte_pairs(v[0], v[1], p);
     return fma_pairs_exact(p, s, c);
   }
 };
