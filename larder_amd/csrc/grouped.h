@@ -233,10 +233,12 @@ __device__ __forceinline__ void dma_a(const _Float16 *ab, uint32_t off, uint32_t
     dma<4>(ab, 0u, lds);
 }
 
-// s_barrier with compiler memory fences on both sides: the intrinsic alone does not order memory accesses, and
-// __syncthreads' release fence would wait for every copy in flight, including the ones meant to stay in flight
+// A barrier that publishes this wavefront's LDS writes and lets other wavefronts overwrite what it has read: its own LDS
+// operations are waited for first (issued is not done: another SIMD's read can pass a write still queued), with compiler
+// memory fences on both sides. __syncthreads' release fence would also wait for every copy in flight, including the ones
+// meant to stay in flight.
 __device__ __forceinline__ void barrier_lds() {
-  asm volatile("" ::: "memory");
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
