@@ -1575,9 +1575,8 @@ extern "C" int lmoe_grouped_tile_rows(void) { return GM; }
 // The tuned tile-row rule (measured on MI355X): 64 when gate/up runs on f16 weights (a type beyond Q4_0 / Q4_K, or
 // gate and up of two types: the f16-weight GEMM then fits two workgroups a CU; 2,048 x 8 rows 405 -> 377 us); 64
 // for a Q4_K gate/up (the direct-copy kernel k_grouped_q4_k_dma: cfg5 gate/up 545 -> 387 us, and as fast as 128
-// rows at 1,000 rows an expert); 128 for a Q4_0 gate/up with an f16 down; 32 when every projection is Q4_0 and an
-// expert averages fewer than 16 rows (batched decode: each tile streams its expert's weights, and 32-row tiles keep
-// five K steps in flight and allow split-K; cfg4 116.6 -> 108.8 us); else 128.
+// rows at 1,000 rows an expert); 128 for a Q4_0 gate/up with an f16 down; by rows an expert when every projection is
+// Q4_0.
 // LMOE_TILE_ROWS and LMOE_KSPLIT override the two rules below (knobs of the kind of the reference's MOE_GGUF_RUN_TILE,
 // gguf_experts.py:590-596, for measuring other tilings). They are read on every call and ignored when the value is
 // not one the GEMMs take for these types: tile rows 32 (Q4 projections only), 64 or 128; split-K 1 to 8 slices that
@@ -1595,8 +1594,12 @@ extern "C" int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u,
   if (!(q4(type_g) && type_u == type_g)) return 64;
   if (type_g == LMOE_Q4_K) return 64;
   if (!q4(type_d)) return GM;
-  const bool all_q4_0 = type_g == LMOE_Q4_0 && type_d == LMOE_Q4_0;
-  return all_q4_0 && E > 0 && (long long)R < 16LL * E ? 32 : GM;
+  // Q4_0 by rows an expert (times on one box, us a layer with 32 / 64 / 128 rows): few rows stream weights through short
+  // tiles, with split-K below (4 rows of 128 experts: 120 / 127 / 139); between, a 64-row tile holds most groups whole
+  // (8: 142 / 133 / 149; 60 experts, 42: 209 / 186 / 204); from 48 up the taller tile decodes a weight for more rows
+  // (64: 242 / 209 / 204; 128: 377 / 309 / 273).
+  if (type_d != LMOE_Q4_0 || E <= 0 || (long long)R >= 48LL * E) return GM;
+  return (long long)R < 6LL * E ? 32 : 64;
 }
 
 // Split-K slices for one grouped GEMM over K: with 32-row tiles and fewer than 16 rows an expert, few tiles have
