@@ -495,8 +495,8 @@ def types_leg():
     """The block types beyond Q4_0 / Q4_K on a cfg2-shaped layer (H 2048, E 128, I 768, top-8), each type for all
     three projections, plus the 35B's Q4_K / Q4_K / Q6_K mix: the decode chain for one token (the general gate/up
     and down kernels, kernel-exact durations against the HBM roofline over the 8 experts' bytes) and the grouped
-    path for 2048 tokens (dequant of the experts to f16, then the f16-weight grouped GEMMs; MFMA roofline over the
-    routed GEMM flops)."""
+    path for 2048 tokens (the grouped GEMMs on the blocks as stored, and on resident f16 weights; MFMA roofline over
+    the routed GEMM flops)."""
     import ctypes
 
     import torch

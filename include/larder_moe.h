@@ -27,7 +27,7 @@ enum { LMOE_Q4_0 = 2, LMOE_Q4_1 = 3, LMOE_Q8_0 = 8, LMOE_Q4_K = 12, LMOE_Q5_K = 
 /* Q4_0 and Q4_K run on every kernel. Q4_1, Q8_0, Q5_K and Q6_K run on the general decode chain
  * (lmoe_gemv_gate_up / lmoe_gemv_down_combine with raw x and float32 h: one lane a 32-weight chunk,
  * gguf_experts.py:78-373's task decoders restated), in lmoe_dequant, and on the grouped path through
- * lmoe_dequant_gemm_f16 + lmoe_grouped_*_f16w; the prepared-row entry points take Q4_0 and Q4_K only. */
+ * lmoe_grouped_*_any or lmoe_dequant_gemm_f16 + lmoe_grouped_*_f16w; the prepared-row entry points take Q4_0 and Q4_K only. */
 /* refusals */
 enum { LMOE_EINVAL = -1, LMOE_ETYPE = -2, LMOE_ESHAPE = -3, LMOE_EALIGN = -4, LMOE_EWORKSPACE = -5 };
 
@@ -274,8 +274,8 @@ int lmoe_grouped_tile_rows(void);
 /* The tuned launch choices for the grouped GEMMs, so every caller makes the same ones (no counterpart in the
  * reference, whose dense path has no tile size; gguf_experts.py:698-722 is the path they serve):
  * lmoe_grouped_pick_tile_rows: the grouping's bm for R rows over E experts with block types (type_g, type_u,
- *   type_d): 64 when gate/up runs on f16 weights (not Q4_0 / Q4_K, or gate and up of two types) or is Q4_K, 128
- *   for a Q4_0 gate/up with an f16 down; with all three Q4_0 32 where R < 6 E, 64 where R < 48 E, else 128;
+ *   type_d): 64 when gate/up is not Q4_0 / Q4_K or of two types, or is Q4_K, 128 for a Q4_0 gate/up with a down
+ *   beyond Q4; with all three Q4_0 32 where R < 6 E, 64 where R < 48 E, else 128;
  * lmoe_grouped_pick_ksplit: split-K slices for one GEMM over K at that bm (4, 3 or 2 for 32-row tiles with
  *   R < 16 E, at least 4 K steps a slice; else 1);
  * lmoe_grouped_workspace_bytes: bytes of the ws that lmoe_grouped_gate_up_bm / lmoe_grouped_down_bm need with
@@ -342,8 +342,8 @@ int lmoe_grouped_down_sl(const void *h, int R, const uint32_t *offsets, const ui
                          int type_d, int n_experts, int I, int H, void *y, int ydtype, void *stream);
 
 /* lmoe_grouped_gate_up / lmoe_grouped_down with f16 weights in the K order (lmoe_dequant_gemm_f16's output:
- * wg16 / wu16 [n_experts][I][H], wd16 [n_experts][H][I]) instead of Q4 blocks: the grouped path of Q4_1, Q8_0,
- * Q5_K and Q6_K experts (the reference's gather_mm on dequantized f16 experts, gguf_experts.py:698-722). Same
+ * wg16 / wu16 [n_experts][I][H], wd16 [n_experts][H][I]) instead of blocks: the grouped path of layers that hold such
+ * copies, of gate and up of two types, and of widths lmoe_grouped_*_any does not take (the reference's gather_mm on dequantized f16 experts, gguf_experts.py:698-722). Same
  * grouping arguments, shapes (I % 128, H % 256 for down, K % 64) and outputs; bm: the grouping's tile rows, 128
  * or 64 (two workgroups a CU). */
 int lmoe_grouped_gate_up_f16w(const void *x, int xdtype, int T, int topk, const uint32_t *order,
@@ -356,9 +356,9 @@ int lmoe_grouped_down_f16w(const void *h, const uint32_t *offsets, const uint32_
 
 /* lmoe_grouped_gate_up_f16w / lmoe_grouped_down_f16w straight from the blocks of one of the types Q4_1, Q8_0, Q5_K and
  * Q6_K (gate and up of one type), decoded inside the GEMM with lmoe_dequant_gemm_f16's roundings: the same results bit
- * for bit without the f16 copies. wg / wu [n_experts][I][row bytes], wd [n_experts][H][row bytes], aligned as that entry takes
- * them (Q5_K 16 bytes, Q4_1 4, else 2); the contracted length a multiple of 128 (256 for Q5_K and Q6_K), I % 128, H % 256 for down; bm 128 or 64. R: down's rows
- * (T topk). Replace the dense path's dequant + gather_mm on these types (gguf_experts.py:698-722; DEQ_SRC :529-539). */
+ * for bit without the f16 copies. wg / wu [n_experts][I][row bytes], wd [n_experts][H][row bytes], aligned as that
+ * entry takes them (Q5_K 16 bytes, Q4_1 4, else 2); the contracted length a multiple of 128 (256 for Q5_K and Q6_K),
+ * I % 128, H % 256 for down; bm 128 or 64. R: down's rows (T topk). Replace the dense path's dequant + gather_mm on these types (gguf_experts.py:698-722; DEQ_SRC :529-539). */
 int lmoe_grouped_gate_up_any(const void *x, int xdtype, int T, int topk, const uint32_t *order,
                              const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles,
                              int bm, const uint8_t *wg, const uint8_t *wu, int type, int n_experts, int H, int I,

@@ -24,7 +24,7 @@ DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 TYPES = {"Q4_0": (2, 32, 18), "Q4_K": (12, 256, 144), "Q4_1": (3, 32, 20), "Q8_0": (8, 32, 34),
          "Q5_K": (13, 256, 176), "Q6_K": (14, 256, 210)}
 # the two types every kernel (prepared rows, fused top-k, nibble-decoding grouped GEMMs) takes; the others run on
-# the general decode chain and on the grouped path over f16-dequantized experts
+# the general decode chain and on the grouped GEMMs that decode any block (or on f16 weights)
 Q4_TYPES = ("Q4_0", "Q4_K")
 
 _P, _I, _SZ, _LL, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_longlong, ctypes.c_float

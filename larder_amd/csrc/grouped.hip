@@ -700,7 +700,7 @@ __global__ void __launch_bounds__(256) k_splitk_finish(const float *ws, int kspl
   }
 }
 
-// ---- f16 weights (the other block types, dequantized in the K order): both operands global -> LDS ---------------
+// ---- f16 weights in the K order (resident copies; widths or mixes k_grouped_any does not take): both global -> LDS --
 
 constexpr int kFwDmaW = GN * 128 / 1024 / 4;         // 16-byte weight copies a lane a step (8)
 
@@ -1572,10 +1572,10 @@ using namespace lmoe;
 
 extern "C" int lmoe_grouped_tile_rows(void) { return GM; }
 
-// The tuned tile-row rule (measured on MI355X): 64 when gate/up runs on f16 weights (a type beyond Q4_0 / Q4_K, or
-// gate and up of two types: the f16-weight GEMM then fits two workgroups a CU; 2,048 x 8 rows 405 -> 377 us); 64
+// The tuned tile-row rule (measured on MI355X): 64 when gate/up is of a type beyond Q4_0 / Q4_K or of two types (on
+// the blocks or on f16 weights, two workgroups then fit a CU; f16 weights, 2,048 x 8 rows: 405 -> 377 us); 64
 // for a Q4_K gate/up (the direct-copy kernel k_grouped_q4_k_dma: cfg5 gate/up 545 -> 387 us, and as fast as 128
-// rows at 1,000 rows an expert); 128 for a Q4_0 gate/up with an f16 down; by rows an expert when every projection is
+// rows at 1,000 rows an expert); 128 for a Q4_0 gate/up with a down beyond Q4; by rows an expert when every projection is
 // Q4_0.
 // LMOE_TILE_ROWS and LMOE_KSPLIT override the two rules below (knobs of the kind of the reference's MOE_GGUF_RUN_TILE,
 // gguf_experts.py:590-596, for measuring other tilings). They are read on every call and ignored when the value is
@@ -1589,8 +1589,8 @@ static int env_knob(const char *name) {
 extern "C" int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u, int type_d) {
   auto q4 = [](int t) { return t == LMOE_Q4_0 || t == LMOE_Q4_K; };
   const int want = env_knob("LMOE_TILE_ROWS");
-  const bool f16w = !(q4(type_g) && type_u == type_g) || !q4(type_d);  // a GEMM on dequantized f16 weights
-  if (want == GM || want == 64 || (want == 32 && !f16w)) return want;
+  const bool beyond = !(q4(type_g) && type_u == type_g) || !q4(type_d);  // a GEMM with no 32-row form
+  if (want == GM || want == 64 || (want == 32 && !beyond)) return want;
   if (!(q4(type_g) && type_u == type_g)) return 64;
   if (type_g == LMOE_Q4_K) return 64;
   if (!q4(type_d)) return GM;

@@ -117,7 +117,8 @@ def from_kperm(h):
 
 def gemm_weights(w, t):
     """Every expert of w [E, rows, row bytes] in ggml type t as f16 [E, rows, cols] in the GEMMs' K order
-    (lmoe_dequant_gemm_f16): the weight operand of the grouped path for the types beyond Q4_0 / Q4_K."""
+    (lmoe_dequant_gemm_f16): the weight operand of the f16-weight GEMMs: resident copies, gate and up of
+    two types, rows _decodes_in_gemm refuses."""
     E, rows = w.shape[0], w.shape[1]
     _, be, bb = _lib.TYPES[t]
     cols = w.shape[2] // bb * be
@@ -159,8 +160,9 @@ def gate_up(x, G, topk, wg, wu, types, h, xh=None, prepped=False, ws=None, kspli
     over the grouping G of x's rows (row p reads x[order[p] // topk]); x [T, H] in natural order, any float dtype,
     meets the weights as f16 in the K order (converted into ``xh``; prepped: x already is that form). Weights are
     decoded inside the GEMM; gate and up of two types, or rows of a type beyond Q4_0 / Q4_K that do not split in steps
-    of 128 weights, are dequantized to f16 first (gemm_weights). ksplit (None: pick_ksplit) and ws (the split-K workspace, allocated when not given) drive split-K. sl: (gate, up) in the
-    stream layout (stream_copy) to read instead of wg / wu, same results bit for bit."""
+    of 128 weights, are dequantized to f16 first (gemm_weights). ksplit (None: pick_ksplit) and ws (the split-K
+    workspace, allocated when not given) drive split-K. sl: (gate, up) in the stream layout (stream_copy) to read
+    instead of wg / wu, same results bit for bit."""
     tg, tu = qcode(types[0]), qcode(types[1])
     if not prepped:
         x = as_gemm_f16(x, xh)

@@ -1,0 +1,23 @@
+"""The tile-row rule of an all-Q4_0 layer at its lines (lmoe_grouped_pick_tile_rows, a host function): 32 rows below 6
+rows an expert, 64 below 48, else 128. The GEMMs give the same bits at every tile height (test_gpu_grouped.py)."""
+import pytest
+
+from larder_amd import _lib
+
+
+@pytest.mark.parametrize("E", (1, 60, 128, 512))
+@pytest.mark.parametrize("rows,off,want", ((6, -1, 32), (6, 0, 64), (48, -1, 64), (48, 0, 128)))
+def test_q4_0_tile_rows_at_the_lines(built_lib, monkeypatch, E, rows, off, want):
+    monkeypatch.delenv("LMOE_TILE_ROWS", raising=False)
+    q = _lib.qcode("Q4_0")
+    assert built_lib.lmoe_grouped_pick_tile_rows(rows * E + off, E, q, q, q) == want
+    # no split-K past the 32-row tiles
+    if want != 32:
+        assert built_lib.lmoe_grouped_pick_ksplit(rows * E + off, E, want, 2048) == 1
+
+
+@pytest.mark.parametrize("R,E,want", ((0, 128, 32), (1, 1, 32), (2 ** 31 - 1, 1, 128), (2 ** 31 - 1, 2 ** 30, 32)))
+def test_q4_0_tile_rows_at_the_ends(built_lib, monkeypatch, R, E, want):
+    monkeypatch.delenv("LMOE_TILE_ROWS", raising=False)
+    q = _lib.qcode("Q4_0")
+    assert built_lib.lmoe_grouped_pick_tile_rows(R, E, q, q, q) == want
