@@ -12,7 +12,7 @@
 //     K, f16: x gathered through the grouped order, or the grouped h rows) goes through LDS, shared by the four.
 //     The weights reach LDS as raw Q4 bytes (Q4_0) or as one nibble word per (MFMA K slice, lane group) plus
 //     scales (Q4_K), and each MFMA lane decodes its own 8 weights to f16 in registers, straight into the MFMA's
-//     weight operand: w = fma(q, d, -8 d) for Q4_0, fma(q, d sc, -dmin m) for Q4_K, q from one fp8 conversion a pair;
+//     weight operand: w = ((1024 + q) - 1032) d for Q4_0, fma(q, d sc, -dmin m) for Q4_K;
 //   * the K order. Inside every 32-wide block of K the GEMMs take the elements in the order
 //     0-3, 16-19, 4-7, 20-23, 8-11, 24-27, 12-15, 28-31 (kperm): then MFMA lane group g's 8 weights are the low
 //     and high nibbles of qs bytes 4g..4g+3, one Q4 word. x comes in that order (lmoe_to_gemm_f16), gate/up writes
@@ -114,7 +114,7 @@ __device__ __forceinline__ Q0Lane q0_lane(int wave, int fr, int g) {
 
 // One K step of a wavefront out of the Q4_0 stage at st into acc. The MFMA order is written out by hand. The
 // step's 8 weight fragments (K slice ks = i / 4, fragment nb = i % 4) go in turn; fragment i's 8 MFMAs issue in
-// pairs with a quarter of fragment i + 1's decode (2-4 VALU) between pairs, so the decode issues while the matrix
+// pairs with a quarter of fragment i + 1's decode (4 VALU) between pairs, so the decode issues while the matrix
 // core works; fragment i + 2's weight word is read from LDS one fragment ahead of its decode and the second K
 // slice's A fragments two fragments ahead of their use. sched_barrier keeps the compiler from regrouping them.
 // QN: the 32-row pairs of fragments the tile has rows in (a tile's last m-tile is often short): the MFMAs and A
@@ -126,6 +126,7 @@ __device__ __forceinline__ void q0_mfma_step(const uint8_t *sa, Word word, Scale
                                              f32x4 (&acc)[4][MB]) {
   __builtin_amdgcn_s_setprio(1);  // the other workgroup's wavefront on this SIMD yields while this one multiplies
   const u32x4 *as = reinterpret_cast<const u32x4 *>(sa);
+  const h2_t bias = {_Float16(1032.0f), _Float16(1032.0f)};
   half8 xf[2][8];
 #pragma unroll
   for (int mb = 0; mb < 2 * QN; ++mb) xf[0][mb] = __builtin_bit_cast(half8, as[achunk(16 * mb + fr, g)]);
@@ -148,7 +149,7 @@ __device__ __forceinline__ void q0_mfma_step(const uint8_t *sa, Word word, Scale
     }
     const int n = i + 1 < 8 ? i + 1 : 7;  // the next fragment (a repeat of the last, unused, after it)
     const _Float16 d = __builtin_bit_cast(h2_t, sw[n])[n / 4];
-    const _Float16 m8d = d * _Float16(-8.0f);  // w = fma(q, d, -8 d), as decode8
+    const h2_t dd = {d, d};
     uint32_t lo = 0, hi = 0;
     u32x4 wnext;
 #pragma unroll
@@ -164,9 +165,8 @@ __device__ __forceinline__ void q0_mfma_step(const uint8_t *sa, Word word, Scale
           lo = xw[n] & 0x0F0F0F0Fu;
           hi = (xw[n] >> 4) & 0x0F0F0F0Fu;
         }
-        const uint32_t n4 = q < 2 ? lo : hi;
-        const h2_t p = q % 2 == 0 ? nibbles_f16<false>(n4) : nibbles_f16<true>(n4);
-        wnext[q] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(p, h2_t{d, d}, h2_t{m8d, m8d}));
+        const uint32_t p = magic_pair(q < 2 ? lo : hi, q % 2 == 0 ? kSel01 : kSel23);
+        wnext[q] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2_t, p) - bias) * dd);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
