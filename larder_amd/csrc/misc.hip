@@ -1,7 +1,5 @@
 // Smaller kernels around the path: the weighted combine of grouped rows, the dequant of whole experts, and a
 // Q4_0 quantizer used to build synthetic packs on the device.
-#include <type_traits>
-
 #include "lmoe_common.h"
 
 namespace lmoe {
@@ -9,7 +7,8 @@ namespace lmoe {
 // out[t][n] = sum_j scores[t][j] y[inv[t k + j]][n] (+ sigmoid(gate) shared) (+ residual), in that order of
 // additions; inv null: row t k + j. VEC: 8 consecutive n a thread (H % 8 == 0, aligned rows), grid (ceil(H / 2048), T);
 // else one n a thread, grid (ceil(H / 256), T). Bound by y's bytes at a prompt's size (8,192 tokens x 8 rows of 2048:
-// 58 us, 5.2 TB/s) and by its round trips at a few tokens, so the rows' loads go out 8 (then 4, 2, 1) at a time.
+// 59 us, 5.2 TB/s). One row a turn: with 8 rows' loads out at once a thread holds 40 VGPRs instead of 12, and a prompt
+// takes 64.5 us for nothing at few tokens.
 template <bool VEC>
 __global__ void __launch_bounds__(256)
     k_combine_sorted(const void *y, int ydt, const uint32_t *inv, const float *scores, int k, int H,
@@ -28,28 +27,15 @@ __global__ void __launch_bounds__(256)
   float acc[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) acc[i] = 0.0f;
-  auto rows = [&](int j0, auto nc) {  // rows j0 .. j0 + N - 1
-    constexpr int N = decltype(nc)::value;
-    float v[N][NV], s[N];
-    size_t row[N];
+  for (int j = 0; j < k; ++j) {
+    const size_t at = size_t(t) * k + j;
+    const size_t row = inv ? inv[at] : at;
+    const float sc = scores ? scores[at] : 1.0f;
+    float v[NV];
+    load(y, row * H + n, ydt, v);
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const size_t at = size_t(t) * k + j0 + j;
-      row[j] = inv ? inv[at] : at;
-      s[j] = scores ? scores[at] : 1.0f;
-    }
-#pragma unroll
-    for (int j = 0; j < N; ++j) load(y, row[j] * H + n, ydt, v[j]);
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-#pragma unroll
-      for (int i = 0; i < NV; ++i) acc[i] = fmaf(s[j], v[j][i], acc[i]);
-  };
-  int j = 0;
-  for (; j + 8 <= k; j += 8) rows(j, std::integral_constant<int, 8>{});
-  if (k - j >= 4) rows(j, std::integral_constant<int, 4>{}), j += 4;
-  if (k - j >= 2) rows(j, std::integral_constant<int, 2>{}), j += 2;
-  if (k - j >= 1) rows(j, std::integral_constant<int, 1>{});
+    for (int i = 0; i < NV; ++i) acc[i] = fmaf(sc, v[i], acc[i]);
+  }
   const size_t o = size_t(t) * H + n;
   if (shared) {
     const float gs = sigmoidf_(load_elt(gate, size_t(t) * gate_stride, gdt));
