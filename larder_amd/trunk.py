@@ -51,8 +51,8 @@ def shared_expert_rows(x, gate, up, down):
         K, N = x.shape[-1], wg.shape[0]
         x2 = x.reshape(-1, K).contiguous()
         h = torch.empty((x2.shape[0], N), dtype=torch.bfloat16, device=x.device)
-        call("lmoe_qmv_swiglu_rows", ptr(x2), x2.shape[0], *(ptr(t.contiguous()) for t in (wg, sg, bg, wu, su, bu)), N, K, gs,
-             ptr(h), stream())
+        held = [t.contiguous() for t in (wg, sg, bg, wu, su, bu)]  # strided ones' copies, alive until the launch is out
+        call("lmoe_qmv_swiglu_rows", ptr(x2), x2.shape[0], *map(ptr, held), N, K, gs, ptr(h), stream())
         return qmv_rows(h.reshape(x.shape[:-1] + (N,)), *down)
     g = qmv_rows(x, *gate)
     u = qmv_rows(x, *up)

@@ -30,6 +30,24 @@ def test_qmv_swiglu_same_bits(T, N, K, G):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+def _column_slices(w):
+    """An affine weight's tensors as column slices of wider buffers."""
+    wide = [torch.cat([t, t.flip(0)[:, :8]], 1)[:, :t.shape[1]] for t in w[:3]]
+    assert not any(t.is_contiguous() for t in wide)
+    return (*wide, w[3])
+
+
+def test_shared_expert_rows_of_strided_weights():
+    """Weights, scales and biases of gate and up that are column slices: the contiguous call's bits."""
+    from larder_amd import trunk
+    rng = np.random.default_rng(11)
+    gate, up, down = _weight(rng, 256, 512, 64), _weight(rng, 256, 512, 64), _weight(rng, 512, 256, 64)
+    x = torch.from_numpy(rng.standard_normal((5, 512)).astype(np.float32)).cuda().bfloat16()
+    want = trunk.shared_expert_rows(x, gate, up, down)
+    got = trunk.shared_expert_rows(x, _column_slices(gate), _column_slices(up), down)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("T,E,k", [(1, 256, 8), (5, 512, 10), (4, 60, 4), (67, 9, 9), (3, 1024, 32)])
 def test_probs_is_topk_reversed(T, E, k):
     from larder_amd import route
