@@ -48,6 +48,15 @@ def test_shared_expert_rows_of_strided_weights():
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+def test_qmv_rows_of_strided_weights():
+    from larder_amd import trunk
+    rng = np.random.default_rng(12)
+    w = _weight(rng, 96, 512, 64)
+    x = torch.from_numpy(rng.standard_normal((5, 512)).astype(np.float32)).cuda().bfloat16()
+    want, got = trunk.qmv_rows(x, *w), trunk.qmv_rows(x, *_column_slices(w))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("T,E,k", [(1, 256, 8), (5, 512, 10), (4, 60, 4), (67, 9, 9), (3, 1024, 32)])
 def test_probs_is_topk_reversed(T, E, k):
     from larder_amd import route

@@ -50,3 +50,9 @@ def test_shared_expert_rows_holds_its_copies(launches):
     x = _wide(torch.zeros((3, 64), dtype=torch.bfloat16))
     trunk.shared_expert_rows(x, _affine(32, 64, 32), _affine(32, 64, 32), _affine(64, 32, 32, wide=False))
     assert launches == ["lmoe_qmv_swiglu_rows", "lmoe_qmv_rows"]
+
+
+def test_qmv_rows_holds_its_copies(launches):
+    x = _wide(torch.zeros((3, 64), dtype=torch.bfloat16))
+    trunk.qmv_rows(x, *_affine(32, 64, 32))
+    assert launches == ["lmoe_qmv_rows"]
