@@ -150,8 +150,9 @@ def stream_copy(w, t):
     cols = w.shape[2] // _lib.TYPES[t][2] * _lib.TYPES[t][1]
     if t not in _lib.Q4_TYPES or _lib.lib().lmoe_stream_bytes(qcode(t), E, rows, cols) == 0:
         raise ValueError(f"{t} experts of {rows} x {cols} have no stream layout (Q4_0 / Q4_K, rows a multiple of 128)")
+    w = w.contiguous()  # a strided w's copy, alive until the launch is out
     out = torch.empty_like(w)
-    call("lmoe_stream_repack", ptr(w.contiguous()), qcode(t), E, rows, cols, ptr(out), stream())
+    call("lmoe_stream_repack", ptr(w), qcode(t), E, rows, cols, ptr(out), stream())
     return out
 
 

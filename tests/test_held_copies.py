@@ -5,7 +5,7 @@ import weakref
 import pytest
 import torch
 
-from larder_amd import trunk
+from larder_amd import grouped, trunk
 
 
 def _wide(t):
@@ -39,7 +39,7 @@ def launches(monkeypatch):
         held.clear()
         names.append(name)
 
-    for module in (trunk,):
+    for module in (grouped, trunk):
         monkeypatch.setattr(module, "ptr", ptr)
         monkeypatch.setattr(module, "call", call)
         monkeypatch.setattr(module, "stream", lambda: None)
@@ -56,3 +56,8 @@ def test_qmv_rows_holds_its_copies(launches):
     x = _wide(torch.zeros((3, 64), dtype=torch.bfloat16))
     trunk.qmv_rows(x, *_affine(32, 64, 32))
     assert launches == ["lmoe_qmv_rows"]
+
+
+def test_stream_copy_holds_its_copy(built_lib, launches):
+    grouped.stream_copy(_wide(torch.zeros((2, 128, 2048 // 32 * 18), dtype=torch.uint8)), "Q4_0")
+    assert launches == ["lmoe_stream_repack"]
