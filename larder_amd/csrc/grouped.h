@@ -125,8 +125,8 @@ __device__ __forceinline__ uint32_t pack_bf2(float a, float b) {
 //   * down, 16-bit: fragments nb and nb + 1 meet through one permlane16 swap a word: lane group g then holds 8
 //     consecutive features, of fragment nb + (g & 1), from 8 (g >> 1) on, so a row's 32 features of the pair go out
 //     as one 64-byte run; f32: each fragment's 4 features as they are.
-// Down rows go to row p of out (grouped order), or with `order` to row order[p] (the caller's order, -0 stored as +0 as a
-// sum over one row's output would give it).
+// Down rows go to row p of out (grouped order), or with `order` to row order[p] (the caller's order; a zero is stored as
+// +0, also where a negative sum rounds to it in f16, as a sum over one row's output in out's dtype would give it).
 // Called by every lane of the workgroup (the swaps read the lanes 16 away); rows past the tile's end store nothing.
 template <int MODE, bool ROWS, int MB>
 __device__ __forceinline__ void store_tile_as(f32x4 (&acc)[4][MB], const Tile &t, int wave, int fr, int g, void *out,
@@ -160,7 +160,12 @@ __device__ __forceinline__ void store_tile_as(f32x4 (&acc)[4][MB], const Tile &t
                                      4 * g) = acc[nb][mb];
       }
     } else {
-      auto pack = [&](float a, float b) { return ROWS && odt == LMOE_BF16 ? pack_bf2(a, b) : pack_h2(a, b); };
+      auto pack = [&](float a, float b) {
+        if (ROWS && odt == LMOE_BF16) return pack_bf2(a, b);
+        h2_t v = {_Float16(a), _Float16(b)};
+        if (ROWS) v += h2_t{_Float16(0.0f), _Float16(0.0f)};
+        return __builtin_bit_cast(uint32_t, v);
+      };
 #pragma unroll
       for (int pr = 0; pr < 2; ++pr) {
         const int nb = 2 * pr;

@@ -694,7 +694,11 @@ __global__ void __launch_bounds__(256) k_splitk_finish(const float *ws, int kspl
   } else if (odt == LMOE_BF16) {
     *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(out) + o + n) = u32x2{pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
   } else {
-    const h2_t v01 = {_Float16(a[0]), _Float16(a[1])}, v23 = {_Float16(a[2]), _Float16(a[3])};
+    h2_t v01 = {_Float16(a[0]), _Float16(a[1])}, v23 = {_Float16(a[2]), _Float16(a[3])};
+    if (order) {  // a zero as +0, as store_tile stores the caller's rows
+      v01 += h2_t{_Float16(0.0f), _Float16(0.0f)};
+      v23 += h2_t{_Float16(0.0f), _Float16(0.0f)};
+    }
     *reinterpret_cast<u32x2 *>(static_cast<_Float16 *>(out) + o + n) =
         u32x2{__builtin_bit_cast(uint32_t, v01), __builtin_bit_cast(uint32_t, v23)};
   }
