@@ -1598,12 +1598,15 @@ extern "C" int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u,
   if (!(q4(type_g) && type_u == type_g)) return 64;
   if (type_g == LMOE_Q4_K) return 64;
   if (!q4(type_d)) return GM;
-  // Q4_0 by rows an expert (times on one box, us a layer with 32 / 64 / 128 rows): few rows stream weights through short
-  // tiles, with split-K below (4 rows of 128 experts: 120 / 127 / 139); between, a 64-row tile holds most groups whole
-  // (8: 142 / 133 / 149; 60 experts, 42: 209 / 186 / 204); from 48 up the taller tile decodes a weight for more rows
-  // (64: 242 / 209 / 204; 128: 377 / 309 / 273).
+  // Q4_0 by rows an expert, swept on the GGUF layout (times on one box, us with 32 / 64 / 128 rows; a layer's): few rows
+  // stream weights through short tiles, with split-K below (4 rows of 128 experts: 120 / 127 / 139); between, a 64-row
+  // tile holds most groups whole (8: 142 / 133 / 149; 60 experts, 42: 209 / 186 / 204); from 48 up the taller tile decodes
+  // a weight for more rows (64: 242 / 209 / 204; 128: 377 / 309 / 273). Few experts leave most of the chip idle without
+  // the split, which 32-row tiles take below 16 rows an expert (gate/up and down alone, 32 / 64: 12 rows of one expert
+  // 2048 x 5632 37 / 98, 15 rows of 8 experts of 1408 42 / 51, of 48 105 / 109, but of 60 120 / 113, of 128 246 / 219).
+  // A folded layer's shared slices count as experts, with every token's row each: the average is what the rule sees.
   if (type_d != LMOE_Q4_0 || E <= 0 || (long long)R >= 48LL * E) return GM;
-  return (long long)R < 6LL * E ? 32 : 64;
+  return (long long)R < (E <= 48 ? 16LL : 6LL) * E ? 32 : 64;
 }
 
 // Split-K slices for one grouped GEMM over K: with 32-row tiles and fewer than 16 rows an expert, few tiles have

@@ -29,9 +29,9 @@ def tile_rows():
 def pick_tile_rows(R, E, types):
     """The GEMMs' tile rows for R rows over E experts (lmoe_grouped_pick_tile_rows, the measured rule): with every
     projection Q4_0, 32 below 6 rows an expert on average (batched decode: few tiles have work, each streams its expert's
-    weights, and 32-row tiles allow split-K), 64 below 48, else 128; 64 when gate/up is of a type beyond Q4_0 / Q4_K, or
-    gate and up of two types, and for Q4_K; otherwise 128. LMOE_TILE_ROWS (32, 64 or 128, read on every call) overrides
-    the rule where the types' GEMMs take that height."""
+    weights, and 32-row tiles allow split-K) or, of at most 48 experts, below 16, 64 below 48, else 128; 64 when gate/up is
+    of a type beyond Q4_0 / Q4_K, or gate and up of two types, and for Q4_K; otherwise 128. LMOE_TILE_ROWS (32, 64 or 128,
+    read on every call) overrides the rule where the types' GEMMs take that height."""
     return _lib.lib().lmoe_grouped_pick_tile_rows(int(R), int(E), *(qcode(t) for t in types))
 
 

@@ -1,19 +1,22 @@
 """The tile-row rule of an all-Q4_0 layer at its lines (lmoe_grouped_pick_tile_rows, a host function): 32 rows below 6
-rows an expert, 64 below 48, else 128. The GEMMs give the same bits at every tile height (test_gpu_grouped.py)."""
+rows an expert (of at most 48 experts below 16, where split-K fills the chip), 64 below 48, else 128. The GEMMs give the
+same bits at every tile height (test_gpu_grouped.py)."""
 import pytest
 
 from larder_amd import _lib
 
 
-@pytest.mark.parametrize("E", (1, 60, 128, 512))
-@pytest.mark.parametrize("rows,off,want", ((6, -1, 32), (6, 0, 64), (48, -1, 64), (48, 0, 128)))
+@pytest.mark.parametrize("E", (1, 8, 48, 49, 60, 128, 512))
+@pytest.mark.parametrize("rows,off,want", (("low", -1, 32), ("low", 0, 64), (48, -1, 64), (48, 0, 128)))
 def test_q4_0_tile_rows_at_the_lines(built_lib, monkeypatch, E, rows, off, want):
     monkeypatch.delenv("LMOE_TILE_ROWS", raising=False)
+    monkeypatch.delenv("LMOE_KSPLIT", raising=False)
     q = _lib.qcode("Q4_0")
+    if rows == "low":
+        rows = 16 if E <= 48 else 6
     assert built_lib.lmoe_grouped_pick_tile_rows(rows * E + off, E, q, q, q) == want
-    # no split-K past the 32-row tiles
-    if want != 32:
-        assert built_lib.lmoe_grouped_pick_ksplit(rows * E + off, E, want, 2048) == 1
+    # split-K up to the line, none past the 32-row tiles
+    assert (built_lib.lmoe_grouped_pick_ksplit(rows * E + off, E, want, 2048) == 1) == (want != 32)
 
 
 @pytest.mark.parametrize("R,E,want", ((0, 128, 32), (1, 1, 32), (2 ** 31 - 1, 1, 128), (2 ** 31 - 1, 2 ** 30, 32)))
