@@ -276,11 +276,14 @@ int lmoe_grouped_tile_rows(void);
  * lmoe_grouped_pick_tile_rows: the grouping's bm for R rows over E experts with block types (type_g, type_u,
  *   type_d): 64 when gate/up is not Q4_0 / Q4_K or of two types, or is Q4_K, 128 for a Q4_0 gate/up with a down
  *   beyond Q4; with all three Q4_0 32 where R < 6 E (E <= 48: R < 16 E), 64 where R < 48 E, else 128;
+ * lmoe_grouped_pick_tile_rows_sl: the same for GEMMs that read stream-layout copies (lmoe_grouped_*_sl): with all
+ *   three Q4_0 32 where R < 40 E, 64 where R < 64 E, else 128;
  * lmoe_grouped_pick_ksplit: split-K slices for one GEMM over K at that bm (4, 3 or 2 for 32-row tiles with
  *   R < 16 E, at least 4 K steps a slice; else 1);
  * lmoe_grouped_workspace_bytes: bytes of the ws that lmoe_grouped_gate_up_bm / lmoe_grouped_down_bm need with
  *   the picked ksplit of each (K = H for gate/up, I for down); 0 when neither splits. */
 int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u, int type_d);
+int lmoe_grouped_pick_tile_rows_sl(int R, int E, int type_g, int type_u, int type_d);
 int lmoe_grouped_pick_ksplit(int R, int E, int bm, int K);
 size_t lmoe_grouped_workspace_bytes(int R, int E, int bm, int H, int I);
 

@@ -66,6 +66,7 @@ SIGNATURES = {
     "lmoe_max_tiles": (_I, [_I, _I, _I]),
     "lmoe_grouped_tile_rows": (_I, []),
     "lmoe_grouped_pick_tile_rows": (_I, [_I, _I, _I, _I, _I]),
+    "lmoe_grouped_pick_tile_rows_sl": (_I, [_I, _I, _I, _I, _I]),
     "lmoe_grouped_pick_ksplit": (_I, [_I, _I, _I, _I]),
     "lmoe_grouped_workspace_bytes": (_SZ, [_I, _I, _I, _I, _I]),
     "lmoe_to_f16": (_I, [_P, _I, _LL, _P, _P]),

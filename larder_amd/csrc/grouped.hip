@@ -1581,7 +1581,7 @@ extern "C" int lmoe_grouped_tile_rows(void) { return GM; }
 // for a Q4_K gate/up (the direct-copy kernel k_grouped_q4_k_dma: cfg5 gate/up 545 -> 387 us, and as fast as 128
 // rows at 1,000 rows an expert); 128 for a Q4_0 gate/up with a down beyond Q4; by rows an expert when every projection is
 // Q4_0.
-// LMOE_TILE_ROWS and LMOE_KSPLIT override the two rules below (knobs of the kind of the reference's MOE_GGUF_RUN_TILE,
+// LMOE_TILE_ROWS and LMOE_KSPLIT override the rules below (knobs of the kind of the reference's MOE_GGUF_RUN_TILE,
 // gguf_experts.py:590-596, for measuring other tilings). They are read on every call and ignored when the value is
 // not one the GEMMs take for these types: tile rows 32 (Q4 projections only), 64 or 128; split-K 1 to 8 slices that
 // divide the K steps, on 32-row tiles of at most 65,535 rows.
@@ -1590,7 +1590,7 @@ static int env_knob(const char *name) {
   return v && *v ? atoi(v) : 0;
 }
 
-extern "C" int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u, int type_d) {
+static int pick_tile_rows(int R, int E, int type_g, int type_u, int type_d, bool stream) {
   auto q4 = [](int t) { return t == LMOE_Q4_0 || t == LMOE_Q4_K; };
   const int want = env_knob("LMOE_TILE_ROWS");
   const bool beyond = !(q4(type_g) && type_u == type_g) || !q4(type_d);  // a GEMM with no 32-row form
@@ -1605,8 +1605,22 @@ extern "C" int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u,
   // the split, which 32-row tiles take below 16 rows an expert (gate/up and down alone, 32 / 64: 12 rows of one expert
   // 2048 x 5632 37 / 98, 15 rows of 8 experts of 1408 42 / 51, of 48 105 / 109, but of 60 120 / 113, of 128 246 / 219).
   // A folded layer's shared slices count as experts, with every token's row each: the average is what the rule sees.
-  if (type_d != LMOE_Q4_0 || E <= 0 || (long long)R >= 48LL * E) return GM;
-  return (long long)R < (E <= 48 ? 16LL : 6LL) * E ? 32 : 64;
+  if (type_d != LMOE_Q4_0 || E <= 0) return GM;
+  const long long r = R, e = E;
+  // On stream copies short tiles pay for longer, and no height splits K: whole runs are copied a tile, so a short tile's
+  // weights cost no more a byte (gate/up and down alone, 32 / 64 / 128 rows: 8 rows of 60 experts 56 / 64 / 70, 15 of 128
+  // 73 / 87 / 104, 28 of 256 121 / 120 / 134, 40 of 128 120 / 118 / 133, 47 of 60 118 / 117 / 125, 64 of 128 161 / 158 / 150).
+  if (stream) return r < 40 * e ? 32 : r < 64 * e ? 64 : GM;
+  if (r >= 48 * e) return GM;
+  return r < (E <= 48 ? 16 : 6) * e ? 32 : 64;
+}
+
+extern "C" int lmoe_grouped_pick_tile_rows(int R, int E, int type_g, int type_u, int type_d) {
+  return pick_tile_rows(R, E, type_g, type_u, type_d, false);
+}
+
+extern "C" int lmoe_grouped_pick_tile_rows_sl(int R, int E, int type_g, int type_u, int type_d) {
+  return pick_tile_rows(R, E, type_g, type_u, type_d, true);
 }
 
 // Split-K slices for one grouped GEMM over K: with 32-row tiles and fewer than 16 rows an expert, few tiles have

@@ -26,13 +26,16 @@ def tile_rows():
     return _lib.lib().lmoe_grouped_tile_rows()
 
 
-def pick_tile_rows(R, E, types):
+def pick_tile_rows(R, E, types, stream=False):
     """The GEMMs' tile rows for R rows over E experts (lmoe_grouped_pick_tile_rows, the measured rule): with every
     projection Q4_0, 32 below 6 rows an expert on average (batched decode: few tiles have work, each streams its expert's
     weights, and 32-row tiles allow split-K) or, of at most 48 experts, below 16, 64 below 48, else 128; 64 when gate/up is
-    of a type beyond Q4_0 / Q4_K, or gate and up of two types, and for Q4_K; otherwise 128. LMOE_TILE_ROWS (32, 64 or 128,
-    read on every call) overrides the rule where the types' GEMMs take that height."""
-    return _lib.lib().lmoe_grouped_pick_tile_rows(int(R), int(E), *(qcode(t) for t in types))
+    of a type beyond Q4_0 / Q4_K, or gate and up of two types, and for Q4_K; otherwise 128. stream: the GEMMs read
+    stream-layout copies, where 32 rows are the fastest below 40 rows an expert and 64 below 64
+    (lmoe_grouped_pick_tile_rows_sl). LMOE_TILE_ROWS (32, 64 or 128, read on every call) overrides the rule where the types'
+    GEMMs take that height."""
+    pick = _lib.lib().lmoe_grouped_pick_tile_rows_sl if stream else _lib.lib().lmoe_grouped_pick_tile_rows
+    return pick(int(R), int(E), *(qcode(t) for t in types))
 
 
 def pick_ksplit(R, E, bm, K):
@@ -65,6 +68,11 @@ class Grouping:
         self.n_tiles = torch.empty(1, **i32)
         nws = _lib.lib().lmoe_group_workspace_bytes(self.R, self.E)
         self.ws = torch.empty(max(nws // 4, 1), **i32)
+
+    def at(self, bm):
+        """This grouping, its next run in m-tiles of bm rows (not below the height it was made with)."""
+        self.bm, self.max_tiles = bm, _lib.lib().lmoe_max_tiles(self.R, self.E, bm)
+        return self
 
     def run(self, ids):
         """Group the flat expert ids [R] (int32 / uint32 on the device); ids >= E go after every expert."""
@@ -273,14 +281,17 @@ class PrefillBuffers:
         self.ids_ext = torch.empty((T, ks), dtype=torch.int32, device=device)
         self.scores_ext = torch.empty((T, ks), **f32)
         self.ids, self.scores = self.ids_ext[:, :L.k], self.scores_ext[:, :L.k]  # the routed picks
-        self.G = Grouping(R, ne, device, bm=pick_tile_rows(R, ne, L.types))
-        nws = splitk_floats(R, ne, self.G.bm, L.H, L.I)
+        # tile rows by the layout the layer's GEMMs read when a pass is made: its blocks as stored, or stream copies
+        self.bm = {sl: pick_tile_rows(R, ne, L.types, sl) for sl in (False, True)}
+        self.G = Grouping(R, ne, device, bm=min(self.bm.values()))
+        nws = splitk_floats(R, ne, self.bm[False], L.H, L.I)
         self.ws = torch.empty(nws, **f32) if nws else None
         self.xh = torch.empty((T, L.H), dtype=torch.float16, device=device)
         self.h = torch.empty((R, L.I), dtype=torch.float16, device=device)
         self.y = torch.empty((R, L.H), dtype=y_dtype, device=device)
         if L.shared is not None and not self.fold:
-            self.Gs = Grouping.identity(T, device, bm=pick_tile_rows(T, 1, L.types))
+            self.Gs, self.Gs_stream = (Grouping.identity(T, device, bm=pick_tile_rows(T, 1, L.types, sl))
+                                       for sl in (False, True))
             self.hs = torch.empty((T, L.Is), dtype=torch.float16, device=device)
             self.ys = torch.empty((T, L.H), **f32)
             # the shared expert runs on a second stream (default priority) beside the routed experts: its dense
@@ -330,7 +341,7 @@ def prefill(layer, x, bufs, out, residual=None, logits=None):
         if not ranked:
             call("lmoe_router_topk_shared", ptr(lg), T, L.E, L.k, int(L.norm), ptr(B.gate), m, ptr(B.ids_ext),
                  ptr(B.scores_ext), st)
-        B.G.run(B.ids_ext.reshape(-1))
+        B.G.at(B.bm[L.folded_stream is not None]).run(B.ids_ext.reshape(-1))
         fs = L.folded_stream or (None, None, None)
         sl_ok = lambda t: t == "Q4_0" or B.G.bm == 64  # noqa: E731
         fg, fu, fd = L.folded
@@ -349,10 +360,11 @@ def prefill(layer, x, bufs, out, residual=None, logits=None):
         with torch.cuda.stream(B.side):
             sg, su, sd = L.shared
             ss = L.shared_stream or (None, None, None)
-            s_ok = lambda t: t == "Q4_0" or B.Gs.bm == 64  # noqa: E731
-            gate_up(B.xh, B.Gs, 1, sg, su, L.types, B.hs, prepped=True,
+            Gs = B.Gs if L.shared_stream is None else B.Gs_stream
+            s_ok = lambda t: t == "Q4_0" or Gs.bm == 64  # noqa: E731
+            gate_up(B.xh, Gs, 1, sg, su, L.types, B.hs, prepped=True,
                     sl=ss[:2] if ss[0] is not None and s_ok(L.types[0]) else None)
-            down(B.hs, B.Gs, sd, L.types[2], B.ys, sl=ss[2] if s_ok(L.types[2]) else None)
+            down(B.hs, Gs, sd, L.types[2], B.ys, sl=ss[2] if s_ok(L.types[2]) else None)
             B.shared_done.record(B.side)
         shared, gate = ptr(B.ys), ptr(B.gate)
     if fused:
@@ -361,7 +373,7 @@ def prefill(layer, x, bufs, out, residual=None, logits=None):
     elif not ranked:
         call("lmoe_router_topk", ptr(lg), _lib.F32, T, L.E, L.k, int(L.norm), ptr(B.ids_ext), ptr(B.scores_ext),
              st)
-    B.G.run(B.ids_ext.reshape(-1))
+    B.G.at(B.bm[L.stream_w is not None]).run(B.ids_ext.reshape(-1))
     f16, sl = L.prefill_f16, L.stream_w or (None, None, None)
     sl_ok = lambda t: t == "Q4_0" or B.G.bm == 64  # noqa: E731  (stream-layout Q4_K: the 64-row kernel)
     gate_up(B.xh, B.G, L.k, L.wg, L.wu, L.types, B.h, prepped=True, ws=B.ws,

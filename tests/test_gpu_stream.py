@@ -126,3 +126,28 @@ def test_prefill_with_stream_copies(cfgid, T, monkeypatch):
     else:
         _, _, want = moe.layer(host(x.float()), host(lg), w, cfg["types"], cfg["k"], cfg["norm"])
     assert moe.rel_l2(host(out), want) < BAR
+
+
+@pytest.mark.parametrize("fold", (True, False))
+def test_stream_copies_take_their_own_tile_rows(fold):
+    """One set of buffers, between the two layouts' lines (21-26 rows an expert, the shared expert apart with 60): 64-row
+    tiles on the blocks as stored, 32-row ones while the layer holds stream copies, whenever they are made; the same bits."""
+    from larder_amd import grouped, workloads
+    from larder_amd import layer as lay
+    cfg = dict(workloads.CONFIGS[1], E=12, I=512, Is=1024)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    L = workloads.make_layer(cfg, g)
+    if not fold:
+        L = lay.MoELayer(L.wg, L.wu, L.wd, L.types, L.k, L.norm, wr=L.wr, shared=L.shared, wsg=L.wsg, fold_shared=False)
+    assert (L.folded is not None) == fold
+    T = 60
+    x = torch.randn((T, cfg["H"]), generator=g, device="cuda").half()
+    B = grouped.PrefillBuffers(L, T)
+    outs, rows = [], []
+    for streamed in (False, True, False):
+        L.keep_stream() if streamed else L.drop_stream()
+        outs.append(torch.empty((T, cfg["H"]), dtype=torch.float32, device="cuda"))
+        grouped.prefill(L, x, B, outs[-1])
+        rows.append(B.G.bm)
+    assert rows == [64, 32, 64]
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
