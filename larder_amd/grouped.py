@@ -141,6 +141,31 @@ def _decodes_in_gemm(t, K, bm):
     return t not in _lib.Q4_TYPES and K % 128 == 0 and bm in (64, tile_rows())
 
 
+# Extra time a step of 128 weights of a 64-row tile, in ns of the whole chip, that decoding a block in the GEMM takes over
+# reading f16 weights
+_DECODE_NS = {"Q4_1": 0.2, "Q8_0": 1.1, "Q5_K": 2.1, "Q6_K": 2.4}
+
+
+def _dequant_pays(t, mats, rows, K, G):
+    """Whether a GEMM over `mats` matrices [E, rows, K] of type t is faster on an f16 copy made first (gemm_weights) than
+    decoding the blocks itself. The copy costs its bytes once, the decode its instructions once a tile of 64 rows, so the
+    copy pays from some 500 (Q6_K) to several thousand (Q4_1) rows an expert on, and for one expert's long rows, whose few
+    workgroups each walk K alone. Both sides are terms in us fitted to a sweep of 16-4,096 rows an expert over 1-512 experts
+    (two boxes; the route taken is 0.8 % off the faster one on average, always decoding 4.1 %). Decode / copy + GEMM:
+      gate/up of 128 experts 768 x 2048: Q6_K 512 rows 841 / 882, 1,024 1,591 / 1,351; Q8_0 1,024 1,357 / 1,386, 2,048
+      2,576 / 2,370; Q5_K 512 796 / 896, 1,024 1,520 / 1,365; Q4_1 2,048 2,292 / 2,283;
+      down of the same: Q6_K 512 493 / 522, 1,024 921 / 781; Q8_0 768 639 / 643, 1,536 1,168 / 1,079;
+      down of one expert 2048 x 5632: Q6_K 16 rows 85 / 61, 256 113 / 87; Q8_0 256 85 / 86.
+    A wide expert's f16 gate and up (8 Mi weights and more a matrix) stream past the caches once a tile and stay on blocks
+    (5632 x 2048, 4,096 rows: Q8_0 335 / 416, Q6_K 402 / 415)."""
+    if mats == 2 and rows * K > 8 << 20:
+        return False
+    if mats == 1 and G.max_tiles * G.bm * K * 2 > 0xFFFFFFFF:  # lmoe_grouped_down_f16w's limit on h
+        return False
+    tiles = max(-(-G.R // 64) * (rows // (128 if mats == 2 else 256)), 320)  # below 320 a tile takes as long as with 320
+    return tiles * (3 + _DECODE_NS[t] * K / 128) * 1e-3 > mats * (8 + 0.86e-6 * G.E * rows * K)
+
+
 def _ws(n, ws, device):
     if n == 0:
         return None
@@ -168,10 +193,10 @@ def gate_up(x, G, topk, wg, wu, types, h, xh=None, prepped=False, ws=None, kspli
     """h [R, I] f16 (grouped order, columns in the GEMMs' K order: from_kperm undoes it) = silu(x . wg) * (x . wu)
     over the grouping G of x's rows (row p reads x[order[p] // topk]); x [T, H] in natural order, any float dtype,
     meets the weights as f16 in the K order (converted into ``xh``; prepped: x already is that form). Weights are
-    decoded inside the GEMM; gate and up of two types, or rows of a type beyond Q4_0 / Q4_K that do not split in steps
-    of 128 weights, are dequantized to f16 first (gemm_weights). ksplit (None: pick_ksplit) and ws (the split-K
-    workspace, allocated when not given) drive split-K. sl: (gate, up) in the stream layout (stream_copy) to read
-    instead of wg / wu, same results bit for bit."""
+    decoded inside the GEMM; gate and up of two types, rows of a type beyond Q4_0 / Q4_K that do not split in steps
+    of 128 weights, and calls where that is faster (_dequant_pays) are dequantized to f16 first (gemm_weights). ksplit
+    (None: pick_ksplit) and ws (the split-K workspace, allocated when not given) drive split-K. sl: (gate, up) in the
+    stream layout (stream_copy) to read instead of wg / wu, same results bit for bit."""
     tg, tu = qcode(types[0]), qcode(types[1])
     if not prepped:
         x = as_gemm_f16(x, xh)
@@ -184,7 +209,8 @@ def gate_up(x, G, topk, wg, wu, types, h, xh=None, prepped=False, ws=None, kspli
         entry, (wg_, wu_) = ("lmoe_grouped_gate_up_sl", sl) if sl is not None else ("lmoe_grouped_gate_up_bm", (wg, wu))
         call(entry, ptr(x), _lib.F16, T, topk, ptr(G.order), ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles),
              G.max_tiles, G.bm, ks, ptr(w), ptr(wg_), ptr(wu_), tg, tu, E, H, I, ptr(h), stream())
-    elif w16 is None and types[0] == types[1] and _decodes_in_gemm(types[0], H, G.bm):
+    elif (w16 is None and types[0] == types[1] and _decodes_in_gemm(types[0], H, G.bm)
+          and not _dequant_pays(types[0], 2, I, H, G)):
         call("lmoe_grouped_gate_up_any", ptr(x), _lib.F16, T, topk, ptr(G.order), ptr(G.offsets), ptr(G.tiles),
              ptr(G.n_tiles), G.max_tiles, G.bm, ptr(wg), ptr(wu), tg, E, H, I, ptr(h), stream())
     else:
@@ -207,7 +233,7 @@ def down(h, G, wd, t, y, ws=None, ksplit=None, w16=None, sl=None):
         call("lmoe_grouped_down_sl" if sl is not None else "lmoe_grouped_down_bm", ptr(h), G.R, ptr(G.offsets),
              ptr(G.tiles), ptr(G.n_tiles), G.max_tiles, G.bm, ks, ptr(w), ptr(sl if sl is not None else wd), qcode(t),
              E, I, H, ptr(y), dcode(y.dtype), stream())
-    elif w16 is None and _decodes_in_gemm(t, I, G.bm):
+    elif w16 is None and _decodes_in_gemm(t, I, G.bm) and not _dequant_pays(t, 1, H, I, G):
         call("lmoe_grouped_down_any", ptr(h), G.R, ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles), G.max_tiles, G.bm,
              ptr(wd), qcode(t), E, I, H, ptr(y), dcode(y.dtype), stream())
     else:
@@ -232,7 +258,9 @@ def expert_rows(x, w, host, types, out_dtype):
     h = torch.empty((R, I), dtype=torch.float16, device=dev)
     out = torch.empty((R, H), dtype=out_dtype, device=dev)
     t = types[2]
-    if t in _lib.Q4_TYPES or _decodes_in_gemm(t, I, G.bm):  # down writes the caller's rows itself
+    # down writes the caller's rows itself, decoding any block: an f16 copy's GEMM, unsorted and masked after, is slower at
+    # every row count (128 experts of 2048 x 768, 2,048 rows each: Q6_K 1,727 against 2,605 us, Q8_0 1,547 against 2,624)
+    if t in _lib.Q4_TYPES or _decodes_in_gemm(t, I, G.bm):
         x = x.contiguous()
         xh = torch.empty((R, H), dtype=torch.float16, device=dev)
         call("lmoe_rows_to_gemm_f16", ptr(x), dcode(x.dtype), R, H, ptr(ids.contiguous()), E, ptr(xh), ptr(out),
