@@ -257,28 +257,19 @@ def expert_rows(x, w, host, types, out_dtype):
     G = Grouping(R, E, dev, bm=pick_tile_rows(R, E, types)).run(ids)
     h = torch.empty((R, I), dtype=torch.float16, device=dev)
     out = torch.empty((R, H), dtype=out_dtype, device=dev)
+    x = x.contiguous()
+    xh = torch.empty((R, H), dtype=torch.float16, device=dev)
+    call("lmoe_rows_to_gemm_f16", ptr(x), dcode(x.dtype), R, H, ptr(ids), E, ptr(xh), ptr(out), dcode(out_dtype), stream())
+    gate_up(xh, G, 1, wg, wu, types, h, prepped=True)
+    # down writes the caller's rows itself, decoding any block: at 60 experts and more an f16 copy's GEMM, unsorted and
+    # masked after, is slower at every row count (128 experts of 2048 x 768, 2,048 rows each: Q6_K 1,727 against 2,605 us,
+    # Q8_0 1,547 against 2,624; one expert of 2048 x 5632, 256 rows: Q6_K 113 against 99, Q8_0 87 against 97)
     t = types[2]
-    # down writes the caller's rows itself, decoding any block: an f16 copy's GEMM, unsorted and masked after, is slower at
-    # every row count (128 experts of 2048 x 768, 2,048 rows each: Q6_K 1,727 against 2,605 us, Q8_0 1,547 against 2,624)
-    if t in _lib.Q4_TYPES or _decodes_in_gemm(t, I, G.bm):
-        x = x.contiguous()
-        xh = torch.empty((R, H), dtype=torch.float16, device=dev)
-        call("lmoe_rows_to_gemm_f16", ptr(x), dcode(x.dtype), R, H, ptr(ids.contiguous()), E, ptr(xh), ptr(out),
-             dcode(out_dtype), stream())
-        gate_up(xh, G, 1, wg, wu, types, h, prepped=True)
-        ks = pick_ksplit(R, E, G.bm, I) if t == "Q4_0" else 1
-        ws = _ws(ks * R * H if ks > 1 else 0, None, dev)
-        call("lmoe_grouped_down_rows", ptr(h), R, ptr(G.order), ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles), G.max_tiles,
-             G.bm, ks, ptr(ws), ptr(wd), qcode(t), E, I, H, ptr(out), dcode(out_dtype), stream())
-        return out
-    # the down GEMM's f32 result goes to out_dtype with one rounding: an f16 y only when out is f16 itself
-    y = torch.empty((R, H), dtype=torch.float16 if out_dtype == torch.float16 else torch.float32, device=dev)
-    gate_up(x.contiguous(), G, 1, wg, wu, types, h)
-    down(h, G, wd, t, y)
-    call("lmoe_combine_sorted", ptr(y), dcode(y.dtype), ptr(G.inv), None, R, 1, H, None, None, 0, None, 0, ptr(out),
-         dcode(out_dtype), stream())
-    bad = (ids < 0) | (ids >= E)
-    return out.masked_fill_(bad[:, None], 0)
+    ks = pick_ksplit(R, E, G.bm, I) if t == "Q4_0" else 1
+    ws = _ws(ks * R * H if ks > 1 else 0, None, dev)
+    call("lmoe_grouped_down_rows", ptr(h), R, ptr(G.order), ptr(G.offsets), ptr(G.tiles), ptr(G.n_tiles), G.max_tiles, G.bm,
+         ks, ptr(ws), ptr(wd), qcode(t), E, I, H, ptr(out), dcode(out_dtype), stream())
+    return out
 
 
 class PrefillBuffers:
