@@ -39,7 +39,8 @@ __device__ __forceinline__ float bf16r(float v) {
 // unless the value is a float32 itself): a value whose rounding to bf16 is the one rounding of the exact value, since
 // only a value that is exactly halfway between two bf16 values ends in 0x8000. The exact value lies between the fused
 // multiply-add rounded down (MODE's round field = 2) and rounded up (1), which are equal or neighbours; the odd one is
-// picked bit by bit. One asm block, so that no other rounding instruction can come between the mode changes; the
+// picked bit by bit. One asm block, so that no other rounding instruction can come between the mode changes (a is written
+// before the last x and w are read, so no input may share its registers); the
 // smallest exact zero keeps the sign that rounding to nearest gives it (rounded up's +0, unless both are -0).
 __device__ __forceinline__ void fma_bf16_odd(float (&a)[16], const float *x, const float *w) {
   float t[16];
@@ -78,8 +79,8 @@ __device__ __forceinline__ void fma_bf16_odd(float (&a)[16], const float *x, con
       "v_fma_f32 %14, %46, %62, %14\n\t"
       "v_fma_f32 %15, %47, %63, %15\n\t"
       "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),
-        "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15]),
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]),
+        "+&v"(a[8]), "+&v"(a[9]), "+&v"(a[10]), "+&v"(a[11]), "+&v"(a[12]), "+&v"(a[13]), "+&v"(a[14]), "+&v"(a[15]),
         "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3]), "=&v"(t[4]), "=&v"(t[5]), "=&v"(t[6]), "=&v"(t[7]),
         "=&v"(t[8]), "=&v"(t[9]), "=&v"(t[10]), "=&v"(t[11]), "=&v"(t[12]), "=&v"(t[13]), "=&v"(t[14]),
         "=&v"(t[15])
