@@ -346,8 +346,9 @@ int lmoe_grouped_down_sl(const void *h, int R, const uint32_t *offsets, const ui
 
 /* lmoe_grouped_gate_up / lmoe_grouped_down with f16 weights in the K order (lmoe_dequant_gemm_f16's output:
  * wg16 / wu16 [n_experts][I][H], wd16 [n_experts][H][I]) instead of blocks: the grouped path of layers that hold such
- * copies, of gate and up of two types, and of widths lmoe_grouped_*_any does not take (the reference's gather_mm on dequantized f16 experts, gguf_experts.py:698-722). Same
- * grouping arguments, shapes (I % 128, H % 256 for down, K % 64) and outputs; bm: the grouping's tile rows, 128
+ * copies, of gate and up of two types, of an H that is an odd multiple of 64 (gate/up), and of calls with so many rows an
+ * expert that a copy made first is faster than decoding the blocks once a tile (the reference's gather_mm on dequantized
+ * f16 experts, gguf_experts.py:698-722). Same grouping arguments, shapes (I % 128, H % 256 for down, K % 64) and outputs; bm: the grouping's tile rows, 128
  * or 64 (two workgroups a CU). */
 int lmoe_grouped_gate_up_f16w(const void *x, int xdtype, int T, int topk, const uint32_t *order,
                               const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles,

@@ -704,7 +704,7 @@ __global__ void __launch_bounds__(256) k_splitk_finish(const float *ws, int kspl
   }
 }
 
-// ---- f16 weights in the K order (resident copies; widths or mixes k_grouped_any does not take): both global -> LDS --
+// ---- f16 weights in the K order (resident copies, gate and up of two types, many rows an expert): both global -> LDS --
 
 constexpr int kFwDmaW = GN * 128 / 1024 / 4;         // 16-byte weight copies a lane a step (8)
 

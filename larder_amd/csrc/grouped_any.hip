@@ -9,13 +9,18 @@
 //     wavefront loads its own 64 rows' bytes into registers two steps ahead, neighbouring lanes on neighbouring bytes of
 //     a row, and writes them to its own part of LDS at their step's start: no barrier waits for weights, and only A has
 //     two stages;
-//   * a lane then reads the words of its 8 weights a slice and decodes them in registers.
+//   * a lane then reads the words of its 8 weights a slice and decodes them in registers;
+//   * a tile is 64 rows: two steps of weights in flight beside 64 accumulators take all 256 VGPRs (32-40 spilled for Q8_0,
+//     20 for Q5_K, 3-7 for Q6_K, none for Q4_1; the reloads stand outside the K loops). A 128-row tile of the grouping is
+//     worked as two, each decoding every weight.
 // Bound: LDS reads and the decode's vector work (15 instructions for 8 weights at Q8_0, ~25 at Q6_K, beside one MFMA for
 // each 16 rows) at many rows an expert, the weights' latency at few. Measured on one box, us for gate/up and down
 // (dequantizing each matrix to f16, 140-158 us each, plus the f16-weight GEMMs -> this kernel):
 //   Q8_0, 3,001 rows, 60 experts of 2048 x 1408          283 + 139 and 142 + 93 -> 127 and 71
 //   Q6_K, 16,384 rows, 128 experts of 2048 x 768         316 + 215 and 158 + 138 -> 278 and 161
 //   Q8_0 / Q6_K, 65,536 rows, the same experts           853 / 886 and 539 / 548 -> 695 / 795 and 485 / 481
+// Past some 500 (Q6_K) to 1,200 (Q8_0) rows an expert the copy is the faster way again, since it is made once and a block
+// is decoded once a tile (262,144 rows, the same experts, Q6_K: 2,350 and 1,325 against 3,043 and 1,736); the caller picks.
 // Loads with each lane on the row its MFMA operand wants (and 4 x 4 word transposes between lane groups in place of LDS)
 // took 221 and 87 us at the first line: neighbouring lanes then look up a cache line each. One step of weights ahead
 // instead of two: 130 and 74, Q4_1 101 and 58 against 91 and 53.
@@ -347,11 +352,12 @@ k_grouped_any(const _Float16 *a_src, int topk, const uint32_t *order, const uint
   store_tile<MODE, MB>(acc, t, wave, fr, g, out, ldo, odt, order);
 }
 
-// Shape checks and the launch both entry points share. mode gate/up: n_rows = I; down: n_rows = H.
+// Shape checks and the launch that lmoe_grouped_gate_up_any, lmoe_grouped_down_any and lmoe_grouped_down_rows share. mode
+// gate/up: n_rows = I; down: n_rows = H.
 int grouped_any(const char *fn, int mode, const void *a, long long a_rows, int topk, const uint32_t *order,
-                       const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles, int bm,
-                       const uint8_t *w0, const uint8_t *w1, int type, int n_experts, int K, int n_rows, void *out,
-                       int odt, hipStream_t st) {
+                const uint32_t *offsets, const uint32_t *tiles, const uint32_t *n_tiles, int max_tiles, int bm,
+                const uint8_t *w0, const uint8_t *w1, int type, int n_experts, int K, int n_rows, void *out, int odt,
+                hipStream_t st) {
   LMOE_REQUIRE(type == LMOE_Q4_1 || type == LMOE_Q8_0 || type == LMOE_Q5_K || type == LMOE_Q6_K, LMOE_ETYPE,
                "%s: ggml type %d is not supported (Q4_1 = 3, Q8_0 = 8, Q5_K = 13, Q6_K = 14)", fn, type);
   LMOE_REQUIRE(bm == GM || bm == 64, LMOE_ESHAPE, "%s: tile rows %d (128 or 64)", fn, bm);

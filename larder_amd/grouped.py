@@ -126,7 +126,7 @@ def from_kperm(h):
 def gemm_weights(w, t):
     """Every expert of w [E, rows, row bytes] in ggml type t as f16 [E, rows, cols] in the GEMMs' K order
     (lmoe_dequant_gemm_f16): the weight operand of the f16-weight GEMMs: resident copies, gate and up of
-    two types, rows _decodes_in_gemm refuses."""
+    two types, rows _decodes_in_gemm refuses, calls where the copy pays (_dequant_pays)."""
     E, rows = w.shape[0], w.shape[1]
     _, be, bb = _lib.TYPES[t]
     cols = w.shape[2] // bb * be
@@ -136,8 +136,8 @@ def gemm_weights(w, t):
 
 
 def _decodes_in_gemm(t, K, bm):
-    """Whether the GEMMs decode type t's blocks themselves over a contraction of K (lmoe_grouped_*_any); else (a row that
-    does not split in steps of 128 weights) the blocks are dequantized to f16 first."""
+    """Whether the GEMMs decode type t's blocks themselves over a contraction of K (lmoe_grouped_*_any); else (an H that is an
+    odd multiple of 64, given to gate_up directly) the blocks are dequantized to f16 first."""
     return t not in _lib.Q4_TYPES and K % 128 == 0 and bm in (64, tile_rows())
 
 

@@ -111,9 +111,10 @@ class MoELayer:
         return self._router_norms
 
     def keep_prefill_f16(self):
-        """Hold the f16 K-order weights the grouped path needs for projections beyond Q4_0 / Q4_K (gate/up together,
-        down alone) resident, so prefill does not dequantize them each call: 2 bytes a weight beside the packed
-        ones, a trade the 288 GB of HBM affords. Returns the bytes held."""
+        """Hold f16 K-order copies of the projections beyond Q4_0 / Q4_K (gate/up together, down alone) resident for the
+        grouped path, so prefill neither decodes their blocks once a tile nor dequantizes them a call (16,384 rows over
+        128 experts of 2048 x 768: Q6_K 391 us against the 500 of dense on blocks, Q8_0 370 against 447): 2 bytes a weight
+        beside the packed ones, a trade the 288 GB of HBM affords. Returns the bytes held."""
         from . import grouped
         gu = None
         if not (self.types[0] in _lib.Q4_TYPES and self.types[1] == self.types[0]):

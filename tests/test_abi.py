@@ -205,10 +205,10 @@ def test_grouped_launch_choices(built_lib):
     assert pick(64 * 8, 128, ("Q4_0",) * 3) == 32         # cfg4 batched decode
     assert pick(2048 * 10, 512, ("Q4_K",) * 3) == 64      # cfg5 prefill: the direct-copy Q4_K kernel
     assert pick(64, 512, ("Q4_K",) * 3) == 64             # few rows, Q4_K
-    assert pick(64, 128, ("Q4_K", "Q4_K", "Q6_K")) == 64   # Q4_K gate/up, f16 down
-    assert pick(64, 128, ("Q4_0", "Q4_0", "Q6_K")) == 128  # Q4_0 gate/up, f16 down
+    assert pick(64, 128, ("Q4_K", "Q4_K", "Q6_K")) == 64   # Q4_K gate/up, a down beyond Q4
+    assert pick(64, 128, ("Q4_0", "Q4_0", "Q6_K")) == 128  # Q4_0 gate/up, a down beyond Q4
     for ts in (("Q8_0",) * 3, ("Q4_0", "Q4_K", "Q4_0"), ("Q6_K", "Q6_K", "Q4_K")):
-        assert pick(2048 * 8, 128, ts) == 64              # gate/up on f16 weights
+        assert pick(2048 * 8, 128, ts) == 64              # gate/up beyond Q4, or of two types
     assert grouped.pick_tile_rows(512, 128, ("Q4_0",) * 3) == 32
     for R, E, bm, K in ((512, 128, 32, 2048), (512, 128, 32, 768), (80, 60, 32, 5632), (512, 128, 32, 256),
                         (512, 128, 128, 2048), (4096, 128, 32, 2048), (16, 4, 32, 192)):
@@ -239,7 +239,7 @@ def test_tile_and_split_knobs(built_lib, monkeypatch):
         assert pick(8192 * 8, 128, q40) == want, v
     monkeypatch.setenv("LMOE_TILE_ROWS", "32")
     assert pick(2048 * 10, 512, q4k) == 32                  # Q4_K has 32-row tiles too
-    assert pick(64, 128, mix) == 64                          # an f16-weight down has none: the rule
+    assert pick(64, 128, mix) == 64                          # a down beyond Q4 has none: the rule
     monkeypatch.setenv("LMOE_TILE_ROWS", "128")
     assert pick(64, 128, mix) == 128
     monkeypatch.delenv("LMOE_TILE_ROWS")

@@ -69,7 +69,7 @@ def test_probs_is_topk_reversed(T, E, k):
 @pytest.mark.parametrize("k", [1, 2, 3, 7, 8, 11, 15, 16])
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
 def test_tail_every_row_count_and_dtype(k, dt):
-    """Any count of rows a token (groups of 8, 4, 2 and 1), aligned and odd widths, shared rows and gates in any dtype."""
+    """Any count of rows a token, aligned and odd widths, shared rows and gates in y's dtype."""
     from larder_amd import route
     g = torch.Generator(device="cuda").manual_seed(k)
     r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
@@ -81,3 +81,23 @@ def test_tail_every_row_count_and_dtype(k, dt):
             w = want if shared is None else want + torch.sigmoid(gate.double()) * sh.double()
             got = route.tail(y, sc, shared, None if shared is None else gate).double()
             assert float((got - w).norm() / w.norm()) < tol
+
+
+@pytest.mark.parametrize("D", [64, 33])
+@pytest.mark.parametrize("y_dt,sh_dt,gate_dt", [(torch.bfloat16, torch.float32, torch.float16),
+                                                (torch.float16, torch.bfloat16, torch.float32),
+                                                (torch.float32, torch.float16, torch.bfloat16),
+                                                (torch.bfloat16, torch.float64, torch.float16),
+                                                (torch.float32, torch.bfloat16, torch.float64)])
+def test_tail_mixed_dtypes(y_dt, sh_dt, gate_dt, D):
+    """y, shared rows and gates of three dtypes (float64 is read as float32): what float32 copies of the two give, bit for
+    bit, and the sum in float64."""
+    from larder_amd import route
+    g = torch.Generator(device="cuda").manual_seed(D)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    y, sc, sh, gate = r(3, 8, D).to(y_dt), r(3, 8), r(3, D).double().to(sh_dt), r(3, 1).double().to(gate_dt)
+    got = route.tail(y, sc, sh, gate)
+    assert got.dtype == y_dt and torch.equal(got, route.tail(y, sc, sh.float(), gate.float()))
+    want = (y.double() * sc.double()[..., None]).sum(-2) + torch.sigmoid(gate.double()) * sh.double()
+    tol = {torch.float32: 1e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[y_dt]  # one rounding of the output
+    assert float((got.double() - want).norm() / want.norm()) < tol

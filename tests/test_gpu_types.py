@@ -2,7 +2,7 @@
 C ABI (larder_amd wrappers): dequant bit for bit (natural order, and the grouped GEMMs' f16 K-order operand to
 f16 rounding), the decode chain (pure and mixed layers such as the 35B's Q4_K / Q4_K / Q6_K, slots past the
 experts giving zero rows), the down + combine epilogue (scores, gated shared expert, residual) and the grouped
-path over dequantized experts, each within the north star's 2e-3 relative L2."""
+path (blocks decoded in the GEMM, or f16 copies), each within 2e-3 relative L2."""
 import numpy as np
 import pytest
 import torch
@@ -118,8 +118,8 @@ def test_down_combine_epilogue(t, k):
                                        (("Q4_K", "Q4_K", "Q6_K"), 1024, 512), (("Q5_K", "Q5_K", "Q5_K"), 1024, 512),
                                        (("Q4_0", "Q4_K", "Q4_0"), 1024, 256)])
 def test_grouped_dense(types, H, I):
-    """gguf_experts.dense over f16-dequantized experts (the f16-weight grouped GEMMs), ragged rows: experts with
-    no rows, one row, and several m-tiles."""
+    """gguf_experts.dense (the GEMMs that decode the blocks; gate and up of two types on f16 copies), ragged rows: experts
+    with no rows, one row, and several m-tiles."""
     from larder_amd import gguf_experts as ge
     rng = np.random.default_rng(H * 3 + I)
     E = 8
@@ -136,9 +136,8 @@ def test_grouped_dense(types, H, I):
 
 
 def test_prefill_with_resident_f16_weights():
-    """A Q4_K / Q4_K / Q6_K layer (and an all-Q8_0 one) through grouped.prefill, dequantizing each call and with
-    keep_prefill_f16's resident weights: the same kernels on the same f16 weights, so the same bits; and against
-    the oracle."""
+    """A Q4_K / Q4_K / Q6_K layer (and an all-Q8_0 one) through grouped.prefill, decoding the blocks in the GEMM and with
+    keep_prefill_f16's resident weights: the same f16 weights either way, so the same bits; and against the oracle."""
     from larder_amd import grouped, layer as lay
     rng = np.random.default_rng(41)
     for types, H, I in ((("Q4_K", "Q4_K", "Q6_K"), 1024, 256), (("Q8_0",) * 3, 1024, 256)):
