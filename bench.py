@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Benchmark: batch-1 decode through a stack of 48 routed-expert MoE layers (BASELINE.json configs[1]) on one
+"""Benchmark: batch-1 decode through a stack of 48 routed-expert MoE layers on one
 MI355X, tokens/s, plus the HBM roofline of the dominant kernel and the CPU baseline beside it.
 
     python bench.py [--steps K] [--warmup W] [--layers 48] [--cpu-seconds 10] [--no-cpu]
@@ -252,7 +252,7 @@ def entry_leg(g):
 
 
 def grouped_leg():
-    """The other configurations (BASELINE.json configs[0] and [2..4]), reported beside the decode line:
+    """The other configurations, reported beside the decode line:
     cfg3 = one 8192-token bf16 prefill chunk through one cfg-2 layer with skewed router logits (MFMA roofline over
     the routed experts' 2 R 3 H I flops); cfg4 = 512 steps of 64 tokens with a fresh Zipf-prior draw each step
     (HBM roofline over the unique experts touched); cfg1 = batch-1 decode through 16 layers with a 5,632-wide shared
@@ -819,7 +819,7 @@ def cpu_configs(cb, secs):
 def main():
     args = parse()
     if args.gpus != 1:
-        print(f"bench.py runs on one GPU: this build has no multi-GPU path (asked for {args.gpus})", file=sys.stderr)
+        print(f"bench.py runs on one GPU: there is no multi-GPU path (asked for {args.gpus})", file=sys.stderr)
         sys.exit(2)
     os.environ.setdefault("HSA_ENABLE_IPC_MODE_LEGACY", "0")
     if args.copy_probe_mib:

@@ -15,7 +15,7 @@ type and ne in the part) followed by a zero "pad" part up to a 4 KiB stride, so 
     fill_slots(packed, key, ids, buf, slots)   records into device slot buffers [S, rows, row bytes]
     load_layer(packed, layer)         a layer's three projections resident in HBM, [E, rows, row bytes] each
 
-The last two are this build's: on a GPU with 288 GB of HBM a whole model's experts (16 GB for the 48-layer
+The last two have no counterpart: on a GPU with 288 GB of HBM a whole model's experts (16 GB for the 48-layer
 Q4_0 stack) stay resident, so the loader streams records through a pinned staging buffer into device tensors the
 expert kernels read directly (the arena slots of the reference's store, stream_fast.py:3936-3941).
 """

@@ -6,7 +6,7 @@ route_cuda.probs / route_cuda.tail (route_cuda.py:280-298) over torch tensors.
     route(gates, mask, slot_of, lam, tau, k, lim=None, slots=True) -> (inds, ok, rhs)   (route_cuda.py:158-178)
     bias_probs(logits, slot_of, lam, tau, k, lim, norm) -> (inds, scores)               (route_cuda.py:306-417)
 
-Differences from the reference kernels, by this build's contract: in probs() ties in the top-k go to the LOWEST
+Differences from the reference kernels, by contract: in probs() ties in the top-k go to the LOWEST
 expert index (route_cuda.py:14-16 breaks them toward the larger one), any E up to 1024 and k up to 32 (not only
 256 / 8), and scores are float32 (the reference rounds them to the logits' bf16). route() and bias_probs() keep the
 reference's rule (larger index) and dtypes, because their callers compare against CacheBiasedMoE's MLX ops. ``inds`` keep the reference's layout: the

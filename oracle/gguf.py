@@ -13,7 +13,7 @@ f16 subnormal d) in tests/test_oracle_props.py.
 The quantizers are not in the reference (it only reads packs that llama.cpp wrote):
   * ``quantize_q4_0`` follows ggml's published ``quantize_row_q4_0_ref`` rule (d = signed-amax / -8,
     q = min(15, trunc(x / d + 8.5))), so it can be checked against ggml's reference behaviour;
-  * ``quantize_q4_k`` is this build's own simple min/scale fit (not ggml's iterative ``make_qkx2_quants``); it
+  * ``quantize_q4_k`` is a plain min/scale fit (not ggml's iterative ``make_qkx2_quants``); it
     only has to produce valid Q4_K blocks from Gaussian weights, and is checked by round trip; the Q4_1, Q5_K,
     Q6_K and Q8_0 quantizers are the same kind of plain fit, checked the same way.
 """

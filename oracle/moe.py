@@ -65,7 +65,7 @@ def router_logits_gemv(x, w):
     thread i of 256 sums, in order, the products of its 8-element items i, i + 256, ... (item j covers elements
     [8 j, 8 j + 8)), starting from zero; each wavefront's 64 partials are added as a balanced binary tree in lane
     order; the four wavefronts' totals are added left to right. Exact for f16 / bf16 inputs, whose products fp32
-    holds without rounding (each step then rounds once, as the GPU's fused multiply-add does); this is this build's
+    holds without rounding (each step then rounds once, as the GPU's fused multiply-add does); this is the router GEMV's
     order, not the reference's: its router is an MLX matmul (stream_fast.py:4352-4356) whose order MLX does not
     fix. Tokens go in chunks and the 256 threads' chains side by side, step by step, so a cfg5
     prefill (2048 tokens, 513 rows of 4096) runs in seconds."""

@@ -11,7 +11,7 @@ stores only data: the blocks fed in and the float32 weights it returned.
 
 Blocks: random bytes with finite f16 scales (as gguf_ref.random_experts makes them, but drawn here), plus edge
 blocks: d = 0, negative d, f16-subnormal d, the largest finite f16 d, +-inf and NaN d (refused by valid()), all-0x00 and all-0xFF nibbles, and blocks
-from this build's own quantizers (oracle.gguf) on Gaussian weights.
+from the oracle's quantizers (oracle.gguf) on Gaussian weights.
 """
 import importlib.util
 import sys

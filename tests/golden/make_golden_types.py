@@ -12,7 +12,7 @@ the build container, never on a GPU box) and stores only data: the blocks fed in
 
 Blocks: random bytes with finite f16 scales, edge blocks (d = 0, negative, f16-subnormal, the largest finite f16,
 +-inf and NaN; all-0x00, all-0xFF and mixed bytes), Q5_K / Q6_K blocks whose scale bytes take every high-bit
-pattern, and blocks from this build's own quantizers (oracle.gguf) on Gaussian weights.
+pattern, and blocks from the oracle's quantizers (oracle.gguf) on Gaussian weights.
 """
 import sys
 from pathlib import Path

@@ -1,4 +1,4 @@
-"""Configuration 5 (BASELINE.json configs[4]): H 4096, 512 routed experts, top-10 renormalised, I 512, a shared
+"""Configuration 5: H 4096, 512 routed experts, top-10 renormalised, I 512, a shared
 expert (Is 512) with a sigmoid gate, all in GGUF Q4_K, at T = 1 (decode chain) and T = 2048 (grouped path); plus the
 device Q4_K quantizer that builds these packs, bit-exact against the CPU oracle's.
 

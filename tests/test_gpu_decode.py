@@ -1,6 +1,6 @@
 """GPU parity of the decode path against the CPU oracle, through the C ABI (larder_amd wrappers).
 
-Bars (BASELINE.json north_star): expert ids and groupings bit-exact, ties to the lowest expert index; layer
+Bars: expert ids and groupings bit-exact, ties to the lowest expert index; layer
 outputs within 2e-3 relative L2 of an fp32 dequant-then-matmul. Quantizer and dequant are integer/byte work and
 must be bit-exact."""
 import numpy as np

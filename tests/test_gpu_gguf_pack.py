@@ -1,6 +1,6 @@
 """Experts packed from a GGUF file and loaded into HBM by larder_amd.gguf_pack feed the expert kernels: the device
 buffers hold the GGUF bytes exactly, and the decode chain and the grouped path on them agree with the CPU oracle
-run on the source tensors (2e-3 relative L2, the north star's bar). Arena-slot filling (fill_slots: experts into
+run on the source tensors (2e-3 relative L2). Arena-slot filling (fill_slots: experts into
 chosen slots of a smaller buffer, in any order) is checked byte for byte."""
 import numpy as np
 import pytest

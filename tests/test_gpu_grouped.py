@@ -1,6 +1,6 @@
 """GPU parity of the grouped (prefill / batched decode) path against the CPU oracle, through the C ABI.
 
-Bars (BASELINE.json north_star): expert ids and groupings bit-exact, ties to the lowest expert index; outputs
+Bars: expert ids and groupings bit-exact, ties to the lowest expert index; outputs
 within 2e-3 relative L2 of an fp32 dequant-then-matmul (oracle.moe). Every row is also held to a per-row bar, so
 one wrong row or tile cannot hide inside a large tensor."""
 import numpy as np
@@ -371,7 +371,7 @@ def test_prefill_cfg3_full_size():
     _, _, want = moe.layer(xs, lgh[sample], tuple(host(b) for b in (L.wg, L.wu, L.wd)), cfg["types"], k,
                            cfg["norm"])
     got = host(out.float())[sample]
-    # the output is bf16: held to the oracle rounded to bf16 the same way, at the north-star bar
+    # the output is bf16: held to the oracle rounded to bf16 the same way, at the same bar
     want_bf16 = host(torch.from_numpy(want.astype(np.float32)).to(torch.bfloat16).float())
     assert moe.rel_l2(got, want_bf16) < BAR
     assert rows_ok(got, want_bf16) < ROW_BAR

@@ -4,7 +4,7 @@ the 35B's Q4_K / Q4_K / Q6_K mix and a Q8_0 down (the prepared chain: gate/up on
 writing h in the Q4_K / Q4_0 order, the Q6_K / Q8_0 down reading it), a Q5_K down (fp32 h, the general down),
 all-Q6_K and Q8_0 gate/up layers (the general gate/up), and given logits.
 Routing is pinned from x (the router GEMV's fixed order restated in the oracle, bit for bit) and the outputs are
-held to the north star's 2e-3 relative L2 against the fp32 dequant-then-matmul oracle."""
+held to 2e-3 relative L2 against the fp32 dequant-then-matmul oracle."""
 import numpy as np
 import pytest
 import torch
