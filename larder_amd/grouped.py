@@ -302,7 +302,7 @@ class PrefillBuffers:
         self.ids, self.scores = self.ids_ext[:, :L.k], self.scores_ext[:, :L.k]  # the routed picks
         # tile rows by the layout the layer's GEMMs read when a pass is made: its blocks as stored, or stream copies
         self.bm = {sl: pick_tile_rows(R, ne, L.types, sl) for sl in (False, True)}
-        self.G = Grouping(R, ne, device, bm=min(self.bm.values()))
+        self.G = Grouping(R, ne, device, bm=min(self.bm.values())).at(self.bm[False])
         nws = splitk_floats(R, ne, self.bm[False], L.H, L.I)
         self.ws = torch.empty(nws, **f32) if nws else None
         self.xh = torch.empty((T, L.H), dtype=torch.float16, device=device)
