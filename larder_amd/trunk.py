@@ -36,8 +36,8 @@ def qmv_rows(x, w, scales, biases, group_size):
     N = w.shape[0]
     x2 = x.reshape(-1, K).contiguous()
     out = torch.empty((x2.shape[0], N), dtype=torch.bfloat16, device=x.device)
-    held = [t.contiguous() for t in (w, scales, biases)]  # strided ones' copies, alive until the launch is out
-    call("lmoe_qmv_rows", ptr(x2), x2.shape[0], *map(ptr, held), N, K, group_size, ptr(out), stream())
+    w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()  # copies live until the launch is out
+    call("lmoe_qmv_rows", ptr(x2), x2.shape[0], ptr(w), ptr(scales), ptr(biases), N, K, group_size, ptr(out), stream())
     return out.reshape(x.shape[:-1] + (N,))
 
 
